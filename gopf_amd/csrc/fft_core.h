@@ -42,8 +42,8 @@ __device__ __forceinline__ cpx<T> mul_i(cpx<T> a) {
 // ---------------------------------------------------------------------------
 // compile-time radix schedules
 // ---------------------------------------------------------------------------
-// V = 0: default schedule; V = 1: low-register schedule (E <= 12) for kernels
-// that keep several transformed lines in registers at once
+// V = 0: default schedule; V = 1: low-register schedule (E <= 8, where the length has one)
+// for kernels that keep several transformed lines in registers at once
 template <int N, int V = 0>
 struct Sched : Sched<N, 0> {};
 #define GPF_SCHED_V(n, v, e, ...)                           \
@@ -65,42 +65,43 @@ GPF_SCHED(128, 16, 8, 16)
 GPF_SCHED(256, 16, 16, 16)
 GPF_SCHED(512, 8, 8, 8, 8)
 GPF_SCHED(1024, 16, 16, 16, 4)
-GPF_SCHED(12, 12, 4, 3)
-GPF_SCHED(24, 24, 8, 3)
-GPF_SCHED(48, 12, 4, 4, 3)
-GPF_SCHED(96, 24, 8, 4, 3)
-GPF_SCHED(192, 24, 8, 8, 3)
-GPF_SCHED(384, 24, 8, 8, 2, 3)
-GPF_SCHED(768, 48, 16, 16, 3)
+// 2^a 3: the factor 3 joins a power of two in one radix (6 = 2 x 3, 12 = 4 x 3, dft_pfa), one
+// exchange fewer than with a radix-3 stage of its own (96^3 FP64 pencils of one array 5.7 -> 4.6 us,
+// with the block rows of k_pencils)
+GPF_SCHED(12, 12, 12)
+GPF_SCHED(24, 12, 4, 6)
+GPF_SCHED(48, 12, 4, 12)
+GPF_SCHED(96, 12, 4, 4, 6)
+GPF_SCHED(192, 12, 4, 4, 12)
+GPF_SCHED(384, 12, 4, 4, 4, 6)
+GPF_SCHED(768, 12, 4, 4, 4, 12)
 GPF_SCHED_V(128, 1, 8, 8, 4, 4)
 GPF_SCHED_V(256, 1, 8, 8, 8, 4)
 GPF_SCHED_V(1024, 1, 8, 8, 8, 4, 4)
-GPF_SCHED_V(24, 1, 12, 4, 2, 3)
-GPF_SCHED_V(96, 1, 12, 4, 4, 2, 3)
-GPF_SCHED_V(192, 1, 12, 4, 4, 4, 3)
-GPF_SCHED_V(384, 1, 12, 4, 4, 4, 2, 3)
-GPF_SCHED_V(768, 1, 12, 4, 4, 4, 4, 3)
-// radix-5 lengths (E = 20 or 10: a multiple of every radix of the schedule)
-GPF_SCHED(80, 20, 4, 4, 5)
-GPF_SCHED(100, 20, 4, 5, 5)
-GPF_SCHED(160, 20, 4, 4, 2, 5)
-GPF_SCHED(200, 20, 4, 2, 5, 5)
-GPF_SCHED(250, 10, 2, 5, 5, 5)
-GPF_SCHED(320, 20, 4, 4, 4, 5)
-GPF_SCHED(400, 20, 4, 4, 5, 5)
-GPF_SCHED(500, 20, 4, 5, 5, 5)
-GPF_SCHED(640, 20, 4, 4, 4, 2, 5)
-GPF_SCHED(800, 20, 4, 4, 2, 5, 5)
-GPF_SCHED(1000, 20, 4, 2, 5, 5, 5)
-GPF_SCHED(1280, 20, 4, 4, 4, 4, 5)
-GPF_SCHED(1600, 20, 4, 4, 4, 5, 5)
-GPF_SCHED(2000, 20, 4, 4, 5, 5, 5)
-GPF_SCHED(2560, 20, 4, 4, 4, 4, 2, 5)
+// radix-5 lengths, the factors 5 joined to powers of two likewise (10 = 2 x 5, 20 = 4 x 5).
+// E = 10 wherever two or three stages allow it: at E = 20 with radices 4 and 5 the FP64 passes
+// spilled (100: 63-76 of 256 VGPRs).  100^3 FP64: update 25.3 -> 14.4 us, rows 18.9 -> 11.8,
+// pencils 16.7 and 18.2 -> 8.2; 400 x 250 FP64: update 19.3 -> 13.7
+GPF_SCHED(80, 20, 4, 20)
+GPF_SCHED(100, 10, 10, 10)
+GPF_SCHED(160, 20, 4, 4, 10)
+GPF_SCHED(200, 10, 2, 10, 10)
+GPF_SCHED(250, 10, 5, 5, 10)
+GPF_SCHED(320, 20, 4, 4, 20)
+GPF_SCHED(400, 20, 20, 20)
+GPF_SCHED(500, 10, 5, 10, 10)
+GPF_SCHED(640, 20, 4, 4, 4, 10)
+GPF_SCHED(800, 20, 4, 10, 20)
+GPF_SCHED(1000, 10, 10, 10, 10)
+GPF_SCHED(1280, 20, 4, 4, 4, 20)
+GPF_SCHED(1600, 20, 4, 20, 20)
+GPF_SCHED(2000, 20, 10, 10, 20)
+GPF_SCHED(2560, 20, 4, 4, 4, 4, 10)
 // radix-7 lengths
 GPF_SCHED(112, 28, 4, 4, 7)
-GPF_SCHED(224, 28, 4, 4, 2, 7)
+GPF_SCHED(224, 28, 4, 4, 14)
 GPF_SCHED(448, 28, 4, 4, 4, 7)
-GPF_SCHED(896, 28, 4, 4, 4, 2, 7)
+GPF_SCHED(896, 28, 4, 4, 4, 14)
 // 2^11 (the largest power of two with a compiled schedule)
 GPF_SCHED(2048, 16, 16, 16, 8)
 GPF_SCHED_V(2048, 1, 8, 8, 8, 8, 4)
@@ -276,6 +277,36 @@ __device__ __forceinline__ void dft16(cpx<T>* a) {
 }
 
 template <int R, int DIR, typename T>
+__device__ __forceinline__ void dftR(cpx<T>* a);
+
+// length P Q with coprime P and Q (Good's prime-factor map, no twiddles between the two):
+// input n = (Q n1 + P n2) mod N, output k with k mod P = k1 and k mod Q = k2, so that
+// exp(2 pi i n k / N) = exp(2 pi i n1 k1 / P) exp(2 pi i n2 k2 / Q)
+template <int P, int Q, int DIR, typename T>
+__device__ __forceinline__ void dft_pfa(cpx<T>* a) {
+    constexpr int N = P * Q;
+    cpx<T> b[N];
+#pragma unroll
+    for (int n2 = 0; n2 < Q; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < P; ++n1) b[n2 * P + n1] = a[(Q * n1 + P * n2) % N];
+        dftR<P, DIR>(&b[n2 * P]);
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < P; ++k1) {
+        cpx<T> c[Q];
+#pragma unroll
+        for (int n2 = 0; n2 < Q; ++n2) c[n2] = b[n2 * P + k1];
+        dftR<Q, DIR>(c);
+#pragma unroll
+        for (int m = 0; m < Q; ++m) {
+            const int k = k1 + P * m;  // every k with k mod P = k1
+            a[k] = c[k % Q];
+        }
+    }
+}
+
+template <int R, int DIR, typename T>
 __device__ __forceinline__ void dftR(cpx<T>* a) {
     if constexpr (R == 2) {
         dft2<DIR>(a[0], a[1]);
@@ -291,6 +322,18 @@ __device__ __forceinline__ void dftR(cpx<T>* a) {
         dft8<DIR>(a);
     } else if constexpr (R == 16) {
         dft16<DIR>(a);
+    } else if constexpr (R == 6) {
+        dft_pfa<2, 3, DIR>(a);
+    } else if constexpr (R == 10) {
+        dft_pfa<2, 5, DIR>(a);
+    } else if constexpr (R == 12) {
+        dft_pfa<4, 3, DIR>(a);
+    } else if constexpr (R == 14) {
+        dft_pfa<2, 7, DIR>(a);
+    } else if constexpr (R == 20) {
+        dft_pfa<4, 5, DIR>(a);
+    } else {
+        static_assert(R == 2, "no register transform of this radix");
     }
 }
 
