@@ -45,6 +45,7 @@
 #include "model.h"
 #include "pointwise.h"
 #include "spectral.h"
+#include "spectral_mid.h"
 
 namespace gpf {
 
@@ -505,16 +506,15 @@ public:
 private:
     // transforms
     const cpx<T>* tw(int n);
-    // stage (optional, inverse passes): the fields' RK4 stage update done as they are loaded
-    // (launch_pencils_stage); src is then unused
-    void pencils(const std::vector<cpx<T>*>& dst, const std::vector<const cpx<T>*>& src, int axis, int dir,
-                 const PencilStageArgs<T>* stage = nullptr);
+    void pencils(const std::vector<cpx<T>*>& dst, const std::vector<const cpx<T>*>& src, int axis, int dir);
     // prog (optional): per input, a dense derived-field program evaluated while loading
-    // instead of reading the input array
+    // instead of reading the input array; last false: the last axis is left untransformed
+    // (the middle pass transforms it)
     void r2c(const std::vector<const T*>& in, const std::vector<cpx<T>*>& out, T in_scale,
-             const std::vector<const DerivedArgs<T>*>* prog = nullptr);
+             const std::vector<const DerivedArgs<T>*>* prog = nullptr, bool last = true);
+    // first false: the arrays are the kscratch ones, already transformed back along the last axis
     void c2r(const std::vector<const cpx<T>*>& in, const std::vector<T*>& out, T scale,
-             const double* add_mean = nullptr, const PencilStageArgs<T>* stage = nullptr);
+             const double* add_mean = nullptr, bool first = true);
     cpx<T>* kscratch(int i);
     T* rscratch(int i);
     // timing
@@ -577,10 +577,20 @@ private:
     // general path
     void general_step_euler();
     void general_step_rk4();
-    void sync_from_spectra(const PencilStageArgs<T>* stage = nullptr);
-    bool fused_stage_args(int stage, PencilStageArgs<T>* out);
+    void sync_from_spectra(bool mid = false);
     void ensure_k_fields();
-    void sync_derived();
+    void sync_derived(bool last = true);
+    // the middle pass (spectral_mid.h) along the last forward axis
+    int mid_axis() const { return g_.ndim == 3 ? 2 : 1; }
+    bool mid_eligible();
+    MidArgs<T> mid_args(int op);
+    void mid_terms(int eq, MidArgs<T>& a, MidField<T>& f, int first = 0);
+    void launch_mid_pass(const MidArgs<T>& a);
+    void mid_rk4_stage(int stage);
+    int mid_ok_ = -1;            // mid_eligible, once known
+    bool mid_cross_ = false;     // some equation reads another field's spectrum
+    bool mid_self_ = false;      // some equation reads a field's spectrum at all
+    bool half_derived_ = false;  // the derived bricks are not transformed along the last axis
     void eval_user_terms_for(int eq);
     void eval_elastic();
     KElasticArgs<T> elastic_args(size_t e) const;
@@ -644,6 +654,9 @@ private:
     std::vector<Buf<T>> stab_;
     bool stab_ok_ = false;
     void build_stage_tables();
+    std::vector<Buf<double>> etab_;  // Euler's factor filt / (1 - dt D) per field, in FP64
+    bool etab_ok_ = false;
+    void build_euler_tables();
     std::vector<Buf<T>> Ktab_;  // K(k) of each elastic term, nk values (built in FP64, stored in T)
     std::vector<Buf<T>> lag_;
     // VolumeConservingLP: indicator brick, field, device state {Multiplier, CurrentIntegral,
@@ -960,11 +973,8 @@ int Engine<T>::pass_times(int maxpass, double* ms, long* launches, char* names, 
 }
 
 template <typename T>
-void Engine<T>::pencils(const std::vector<cpx<T>*>& dst, const std::vector<const cpx<T>*>& src, int axis, int dir,
-                        const PencilStageArgs<T>* stage) {
+void Engine<T>::pencils(const std::vector<cpx<T>*>& dst, const std::vector<const cpx<T>*>& src, int axis, int dir) {
     const int n = (axis == 1) ? g_.ny : g_.nz;
-    if (stage && (dir != 1 || dst.size() > (size_t)kMaxArr))
-        throw Error(GPF_EINVAL, "fused stage pencils: one inverse pass of at most 4 fields");
     for (size_t q0 = 0; q0 < dst.size(); q0 += kMaxArr) {
         PencilArgs<T> a;
         a.tw = tw(n);
@@ -984,21 +994,13 @@ void Engine<T>::pencils(const std::vector<cpx<T>*>& dst, const std::vector<const
                 a.src[q][1] = src[q0 + q] + g_.nmain;
             }
         }
-        if (stage) {
-            if constexpr (sizeof(T) == 8) {
-                PencilStageArgs<T> sa = *stage;
-                sa.p = a;
-                HIPCHK(launch_pencils_stage<T>(sa, n, st_));
-                continue;
-            }
-        }
         HIPCHK(launch_pencils<T>(a, n, dir, st_));
     }
 }
 
 template <typename T>
 void Engine<T>::r2c(const std::vector<const T*>& in, const std::vector<cpx<T>*>& out, T in_scale,
-                    const std::vector<const DerivedArgs<T>*>* prog) {
+                    const std::vector<const DerivedArgs<T>*>* prog, bool last) {
     for (size_t q0 = 0; q0 < in.size(); q0 += kMaxArr) {
         RowR2CArgs<T> a;
         a.tw = tw(g_.nx);
@@ -1022,14 +1024,14 @@ void Engine<T>::r2c(const std::vector<const T*>& in, const std::vector<cpx<T>*>&
         a.in_scale = in_scale;
         HIPCHK(launch_rows_r2c<T>(a, st_));
     }
-    pencils(out, {}, 1, -1);
-    if (g_.ndim == 3) pencils(out, {}, 2, -1);
+    if (last || g_.ndim == 3) pencils(out, {}, 1, -1);
+    if (last && g_.ndim == 3) pencils(out, {}, 2, -1);
 }
 
 template <typename T>
 void Engine<T>::c2r(const std::vector<const cpx<T>*>& in, const std::vector<T*>& out, T scale,
-                    const double* add_mean, const PencilStageArgs<T>* stage) {
-    if (stage && in.size() > (size_t)kMaxArr) throw Error(GPF_EINVAL, "fused stage pencils: at most 4 fields");
+                    const double* add_mean, bool first) {
+    if (!first && in.size() > (size_t)kMaxArr) throw Error(GPF_EINVAL, "half-inverted arrays: at most 4");
     for (size_t q0 = 0; q0 < in.size(); q0 += kMaxArr) {
         const int na = (int)std::min(in.size() - q0, (size_t)kMaxArr);
         std::vector<cpx<T>*> scr;
@@ -1039,10 +1041,10 @@ void Engine<T>::c2r(const std::vector<const cpx<T>*>& in, const std::vector<T*>&
             src.push_back(in[q0 + q]);
         }
         if (g_.ndim == 3) {
-            pencils(scr, src, 2, +1, stage);
+            if (first) pencils(scr, src, 2, +1);
             pencils(scr, {}, 1, +1);
-        } else {
-            pencils(scr, src, 1, +1, stage);
+        } else if (first) {
+            pencils(scr, src, 1, +1);
         }
         RowC2RArgs<T> a;
         a.tw = tw(g_.nx);
@@ -1453,7 +1455,7 @@ void Engine<T>::set_filter(const double* table) {
     if (table && stepper_ == GPF_SDD) throw Error(GPF_EINVAL, "SDD: Does not support modal filters");
     HIPCHK(hipStreamSynchronize(st_));
     drop_graph();
-    stab_ok_ = false;
+    stab_ok_ = etab_ok_ = false;
     if (!table) {
         has_filter_ = false;
         return;
@@ -1461,7 +1463,6 @@ void Engine<T>::set_filter(const double* table) {
     if (!filter_.get()) filter_.alloc(1000);
     HIPCHK(hipMemcpy(filter_.get(), table, 1000 * sizeof(double), hipMemcpyHostToDevice));
     has_filter_ = true;
-    stab_ok_ = false;
 }
 
 template <typename T>
@@ -1892,7 +1893,8 @@ void Engine<T>::ensure_k_fields() {
 }
 
 template <typename T>
-void Engine<T>::sync_derived() {
+void Engine<T>::sync_derived(bool last) {
+    half_derived_ = !last;
     if (nd_ == 0) return;
     std::vector<const T*> in;
     std::vector<cpx<T>*> out;
@@ -1907,7 +1909,7 @@ void Engine<T>::sync_derived() {
         prog.push_back(inline_prog ? &dargs_[d] : nullptr);
         out.push_back(K_[nf_ + d].get());
     }
-    r2c(in, out, T(1), &prog);
+    r2c(in, out, T(1), &prog, last);
 }
 
 // SquaredGradient terms of equation eq, evaluated on the current k-space bricks
@@ -1976,14 +1978,17 @@ void Engine<T>::eval_elastic() {
         ind.dc[2][0] = 3.0;
         ind.dc[3][0] = -2.0;
         const std::vector<const DerivedArgs<T>*> prog{&ind};
-        r2c({nullptr}, {Hk}, T(1), &prog);
-        KElasticArgs<T> a = elastic_args(e);
-        a.src = Hk;
-        a.dst = Hk;
-        a.ktab = Ktab_[e].get();
-        HIPCHK(launch_kelastic<T>(a, st_));
-        if (g_.ndim == 3) pencils({Hk}, {}, 2, +1);
-        pencils({Hk}, {}, 1, +1);
+        // along the last axis: forward, times K(k), back
+        r2c({nullptr}, {Hk}, T(1), &prog, false);
+        MidArgs<T> a = mid_args(kMidScale);
+        a.nf = 1;
+        a.f[0].nterm = 1;
+        a.f[0].t[0].b = Hk;
+        a.f[0].t[0].line = 1;
+        a.f[0].s = Ktab_[e].get();
+        a.f[0].out = Hk;
+        launch_mid_pass(a);
+        if (g_.ndim == 3) pencils({Hk}, {}, 1, +1);
         RowSyncArgs<T> r;
         r.tw = tw(g_.nx);
         r.fmain[0] = Hk;
@@ -2072,20 +2077,128 @@ void Engine<T>::terms_into(int eq, A& a) {
     }
 }
 
+// The middle pass serves equations whose explicit terms are fields, derived fields, constants,
+// elastic terms and volume-conserving terms (at most kMidTerms of them).  A SquaredGradient term
+// is formed from the whole spectra between the passes, and a ConservativeNoise term needs the
+// frequency vector: those keep the separate passes.
+template <typename T>
+bool Engine<T>::mid_eligible() {
+    if (mid_ok_ >= 0) return mid_ok_ == 1;
+    bool ok = nf_ <= kMaxArr;
+    for (int i = 0; i < nf_ && ok; ++i) {
+        ok = eqs_[i].terms.size() <= (size_t)kMidTerms;
+        for (const auto& t : eqs_[i].terms) {
+            ok = ok && t.kind != kSquaredGradient && t.kind != kConservativeNoise;
+            const int b = (t.kind == kConcrete) ? t.brick : (t.kind == kVolumeConserving) ? vc_brick_[t.user] : -1;
+            if (b >= 0 && b < nf_) {
+                mid_self_ = true;
+                mid_cross_ |= b != i;
+            }
+        }
+    }
+    mid_ok_ = ok ? 1 : 0;
+    return ok;
+}
+
+template <typename T>
+MidArgs<T> Engine<T>::mid_args(int op) {
+    MidArgs<T> a;
+    const int axis = mid_axis(), n = axis_len(axis);
+    a.p.tw = tw(n);
+    a.p.seg[0] = (axis == 2) ? seg_z_main(g_) : seg_y_main(g_);
+    a.p.seg[1] = (axis == 2) ? seg_z_nyq(g_) : seg_y_nyq(g_);
+    a.p.nseg = 2;
+    a.p.TW = spread_tw(choose_tw(n, 1, sizeof(cpx<T>), 8, 1, 128),
+                       (long)a.p.seg[0].na * a.p.seg[0].nb + (long)a.p.seg[1].na * a.p.seg[1].nb);
+    a.op = op;
+    a.g = g_.kg;
+    a.nmain = g_.nmain;
+    a.nk = g_.nk;
+    return a;
+}
+
+// the explicit terms of equation eq as terms `first` onwards of f: derived bricks are lines
+template <typename T>
+void Engine<T>::mid_terms(int eq, MidArgs<T>& a, MidField<T>& f, int first) {
+    KUpdateArgs<T> k;
+    terms_into(eq, k);
+    if (first + k.nterm > kMidTerms) throw Error(GPF_EINVAL, "too many terms for the middle pass");
+    f.nterm = first + k.nterm;
+    for (int q = 0; q < k.nterm; ++q) {
+        MidTerm<T>& t = f.t[first + q];
+        t.b = k.brick[q];
+        t.coef = k.coef[q];
+        t.pw = k.pw[q];
+        t.dmul = k.dmul[q];
+        for (int d = 0; d < nd_; ++d) t.line |= (t.b == K_[nf_ + d].get()) ? 1 : 0;
+        a.need_l |= t.pw != 0;
+    }
+}
+
+template <typename T>
+void Engine<T>::launch_mid_pass(const MidArgs<T>& a) {
+    HIPCHK(launch_mid<T>(a, axis_len(mid_axis()), st_));
+}
+
+// Euler's factor filt / (1 - dt D(k)) depends only on the plan: tabulated once, in FP64 at both
+// precisions (a factor rounded to FP32 would be a per-mode error that compounds over the steps)
+template <typename T>
+void Engine<T>::build_euler_tables() {
+    etab_.clear();
+    for (int i = 0; i < nf_; ++i) {
+        etab_.emplace_back(g_.nk);
+        StageDenomArgs<double> a;
+        a.denom = eqs_[i].denom;
+        a.sv = eqs_[i].sv;
+        a.hs = eqs_[i].hs;
+        a.gamma = dt_;
+        a.filter = has_filter_ ? filter_.get() : nullptr;
+        a.g = g_.kg;
+        a.nmain = g_.nmain;
+        a.nk = g_.nk;
+        a.out = etab_.back().get();
+        HIPCHK(launch_stage_denoms<double>(a, st_));
+    }
+    etab_ok_ = true;
+}
+
 template <typename T>
 void Engine<T>::general_step_euler() {
+    const bool mid = mid_eligible();
+    if (mid && !etab_ok_) build_euler_tables();
     ensure_k_fields();
-    sync_derived();
+    sync_derived(!mid);
     eval_elastic();
-    for (int i = 0; i < nf_; ++i) {
-        eval_user_terms_for(i);
-        rhs_update(i, K_[i].get(), K_[i].get(), 1.0, dt_, dt_, true, nullptr);
-    }
     std::vector<const cpx<T>*> in;
     std::vector<T*> out;
     for (int i = 0; i < nf_; ++i) {
         in.push_back(K_[i].get());
         out.push_back(F_[i].get());
+    }
+    if (mid) {
+        // all fields in one launch, or one after the other where an equation reads another
+        // field's spectrum (it then reads the ones before it updated, as euler.go:27-39)
+        const int per = mid_cross_ ? 1 : nf_;
+        for (int i0 = 0; i0 < nf_; i0 += per) {
+            MidArgs<T> a = mid_args(kMidEuler);
+            a.bc = dt_;
+            a.nf = per;
+            for (int q = 0; q < per; ++q) {
+                MidField<T>& f = a.f[q];
+                mid_terms(i0 + q, a, f);
+                f.k = K_[i0 + q].get();
+                f.kn = K_[i0 + q].get();
+                f.s64 = etab_[i0 + q].get();
+                f.out = kscratch(i0 + q);
+            }
+            launch_mid_pass(a);
+        }
+        c2r(in, out, T(1) / (T)g_.n, nullptr, false);
+        return;
+    }
+    for (int i = 0; i < nf_; ++i) {
+        eval_user_terms_for(i);
+        rhs_update(i, K_[i].get(), K_[i].get(), 1.0, dt_, dt_, true, nullptr);
     }
     c2r(in, out, T(1) / (T)g_.n);
 }
@@ -2095,18 +2208,21 @@ void Engine<T>::general_step_euler() {
 // (the last stage writes them).  Used when every derived field is a dense polynomial of
 // the (at most two) fields.
 template <typename T>
-void Engine<T>::sync_from_spectra(const PencilStageArgs<T>* stage) {
+void Engine<T>::sync_from_spectra(bool mid) {
     std::vector<cpx<T>*> scr;
     std::vector<const cpx<T>*> src;
     for (int i = 0; i < nf_; ++i) {
         scr.push_back(kscratch(i));
         src.push_back(K_[i].get());
     }
+    // with the middle pass the scratch arrays hold the fields inverted along the last axis, and
+    // the derived fields are left to it along that axis
+    half_derived_ = mid;
     if (g_.ndim == 3) {
-        pencils(scr, src, 2, +1, stage);
+        if (!mid) pencils(scr, src, 2, +1);
         pencils(scr, {}, 1, +1);
-    } else {
-        pencils(scr, src, 1, +1, stage);
+    } else if (!mid) {
+        pencils(scr, src, 1, +1);
     }
     RowSyncArgs<T> a;
     a.tw = tw(g_.nx);
@@ -2128,8 +2244,8 @@ void Engine<T>::sync_from_spectra(const PencilStageArgs<T>* stage) {
     a.nx = g_.nx;
     a.TW = spread_tw(choose_tw(g_.nx, 1, sizeof(cpx<T>), 1), g_.rows);
     HIPCHK(launch_rows_sync<T>(a, st_));
-    pencils(out, {}, 1, -1);
-    if (g_.ndim == 3) pencils(out, {}, 2, -1);
+    if (!mid || g_.ndim == 3) pencils(out, {}, 1, -1);
+    if (!mid && g_.ndim == 3) pencils(out, {}, 2, -1);
 }
 
 // The factor 1 / (1 - gamma dt D(k)) of RK4's stages depends only on the plan and on gamma
@@ -2161,56 +2277,35 @@ void Engine<T>::build_stage_tables() {
     stab_ok_ = true;
 }
 
-// A stage's update done by the fields' first inverse pencil pass (launch_pencils_stage)
-// instead of its own pass: when every field's equation has at most kStageTerms terms of
-// tmode 0, none formed per stage (SquaredGradient), a stage factor table, and the first
-// inverse axis has a core length.  The pass reads the operands the stage kernel reads and
-// does its arithmetic, so the result is the same; the corrected spectrum is stored only
-// after the last stage (the next step's state) or when an equation reads a field's
-// spectrum as a brick.
+// One RK4 stage as the middle pass: the derived fields' last forward transform, the stage's
+// right-hand side, PrepareNextCorrection and correction (rk4.go:77-127) and the corrected
+// fields' first inverse transform into the scratch arrays.  The corrected spectra are stored only
+// after the last stage (the next step's state) or when an equation reads a field's spectrum;
+// where they are not, K_ keeps the step's initial spectra and no copy of them is made.
 template <typename T>
-bool Engine<T>::fused_stage_args(int stage, PencilStageArgs<T>* out) {
-    if (sizeof(T) != 8 || !stab_ok_ || nf_ > kMaxArr) return false;  // FP64 only (spectral_stage.hip)
-    if (!stage_pencil_length(g_.ndim == 3 ? g_.nz : g_.ny)) return false;
+void Engine<T>::mid_rk4_stage(int stage) {
     const double fac_prep[4] = {1.0 / 6.0, 1.0 / 3.0, 1.0 / 3.0, 1.0 / 6.0};
-    const double fac_corr[3] = {0.5, 0.5, 1.0};
-    PencilStageArgs<T> a;
-    a.stage = stage;
-    a.dt = dt_;
-    a.fp = fac_prep[stage];
-    a.fc = stage < 3 ? fac_corr[stage] : 0.0;
-    a.g = g_.kg;
-    a.nmain = g_.nmain;
-    a.nk = g_.nk;
-    bool field_brick = false;
+    const double fac_corr[4] = {0.5, 0.5, 1.0, 0.0};
+    MidArgs<T> a = mid_args(stage == 0 ? kMidStage0 : stage < 3 ? kMidStage12 : kMidStage3);
+    a.nf = nf_;
+    a.bp = fac_prep[stage] * dt_;
+    a.bc = fac_corr[stage] * dt_;
+    const int kind = (stage < 2) ? 0 : (stage == 3 && has_filter_) ? 2 : 1;
+    const bool store = stage == 3 || mid_self_;
     for (int i = 0; i < nf_; ++i) {
-        for (const auto& t : eqs_[i].terms)
-            if (t.kind == kSquaredGradient || t.kind == kConservativeNoise) return false;
-        Rk4StageArgs<T> r;
-        terms_into(i, r);
-        if (r.nterm > kStageTerms) return false;
-        const int kind = (stage < 2) ? 0 : (stage == 3 && has_filter_) ? 2 : 1;
-        StageLine<T>& f = a.f[i];
-        f.stab = stab_[3 * i + kind].get();
-        if (!f.stab) return false;
+        MidField<T>& f = a.f[i];
+        mid_terms(i, a, f);
         f.k = K_[i].get();
-        f.init = INIT_[i].get();
-        f.final = FINAL_[i].get();
-        f.kn = KF_[i].get();
-        f.nterm = r.nterm;
-        for (int q = 0; q < r.nterm; ++q) {
-            if (r.tmode[q] != 0) return false;
-            f.brick[q] = r.brick[q];
-            f.coef[q] = r.coef[q];
-            f.pw[q] = r.pw[q];
-            f.dmul[q] = r.dmul[q];
-            a.need_l |= (r.pw[q] != 0) ? 1 : 0;
-            for (int j = 0; j < nf_; ++j) field_brick |= (r.brick[q] == K_[j].get());
-        }
+        f.fin = FINAL_[i].get();
+        // the stage's starting values: a copy only where K_ itself changes between the stages
+        f.init = mid_self_ ? INIT_[i].get() : stage == 0 ? nullptr : K_[i].get();
+        f.kn = store ? KF_[i].get() : nullptr;
+        f.s = stab_[3 * i + kind].get();
+        f.out = kscratch(i);
     }
-    a.store_kn = (stage == 3 || field_brick) ? 1 : 0;
-    *out = a;
-    return true;
+    launch_mid_pass(a);
+    if (store)
+        for (int i = 0; i < nf_; ++i) K_[i].swap(KF_[i]);
 }
 
 template <typename T>
@@ -2220,17 +2315,17 @@ void Engine<T>::general_step_rk4() {
     // evaluated from the bricks inside the pass instead of being stored.  The corrected
     // spectra go to KF_ (free, as the right-hand side is never stored) and swap with K_
     // after all fields, so every field of a stage reads the same bricks.  Where possible
-    // (fused_stage_args) that pass is the fields' first inverse pencil pass itself.
+    // (mid_eligible) that pass is the middle pass of the transforms.
+    const bool mid = mid_eligible();
     if (!stab_ok_) build_stage_tables();
     ensure_k_fields();
-    sync_derived();
+    sync_derived(!mid);
     eval_elastic();  // the lagged field is constant within a step (homoLinElast.go:130-134)
     const double fac_prep[4] = {1.0 / 6.0, 1.0 / 3.0, 1.0 / 3.0, 1.0 / 6.0};
     const double fac_corr[3] = {0.5, 0.5, 1.0};
     for (int stage = 0; stage < 4; ++stage) {
-        PencilStageArgs<T> fs;
-        const bool fused = fused_stage_args(stage, &fs);
-        for (int i = 0; i < nf_ && !fused; ++i) {
+        if (mid) mid_rk4_stage(stage);
+        for (int i = 0; i < nf_ && !mid; ++i) {
             eval_user_terms_for(i);
             Rk4StageArgs<T> a;
             terms_into(i, a);
@@ -2258,16 +2353,16 @@ void Engine<T>::general_step_rk4() {
         std::vector<const cpx<T>*> in;
         std::vector<T*> out;
         for (int i = 0; i < nf_; ++i) {
-            K_[i].swap(KF_[i]);
+            if (!mid) K_[i].swap(KF_[i]);
             in.push_back(K_[i].get());
             out.push_back(F_[i].get());
         }
         if (stage < 3 && row_sync_) {
-            sync_from_spectra(fused ? &fs : nullptr);
+            sync_from_spectra(mid);
             continue;
         }
-        c2r(in, out, T(1) / (T)g_.n, nullptr, fused ? &fs : nullptr);
-        if (stage < 3) sync_derived();
+        c2r(in, out, T(1) / (T)g_.n, nullptr, !mid);
+        if (stage < 3) sync_derived(!mid);
     }
 }
 
@@ -2762,7 +2857,12 @@ void Engine<T>::on_step_finished() {
                                    vc_part_.get() + nb, nb, st_));
         const int b = vc_brick_[v];
         const T* ind = (b < nf_) ? F_[b].get() : reinterpret_cast<const T*>(K_[b].get());
-        HIPCHK(launch_volcons_update<T>(vc_part_.get() + nb, nb, ind, ut.dt, vc_state_[v].get(), st_));
+        // a derived brick not transformed along the last axis: its zero mode is the sum of the
+        // line at the other frequencies' zeros
+        const bool line = b >= nf_ && half_derived_;
+        const long cnt = line ? axis_len(mid_axis()) : 1;
+        const long stride = line ? 2 * (mid_axis() == 2 ? seg_z_main(g_) : seg_y_main(g_)).es : 0;
+        HIPCHK(launch_volcons_update<T>(vc_part_.get() + nb, nb, ind, cnt, stride, ut.dt, vc_state_[v].get(), st_));
     }
     for (size_t e = 0; e < lag_.size(); ++e) {
         const UserTerm& ut = mcopy_.user_table[kHomogeneousModulus][e];

@@ -221,7 +221,7 @@ struct KGradArgs {
     long nmain = 0, nk = 0;
 };
 
-// Khachaturyan kernel: dst = K(k) src with K the scalar elastic kernel
+// Khachaturyan kernel: the scalar elastic kernel K(k)
 struct ElasticParams {
     double C[81];
     double sig[9];   // effective stress C : misfit
@@ -229,12 +229,9 @@ struct ElasticParams {
 };
 template <typename T>
 struct KElasticArgs {
-    const cpx<T>* src = nullptr;
-    cpx<T>* dst = nullptr;
     ElasticParams ep;
     KGrid g;
     long nmain = 0, nk = 0;
-    const T* ktab = nullptr;       // K(k), filled once by launch_kelastic_table
 };
 
 // adjoint of the fused semi-implicit step (single field)
@@ -323,14 +320,13 @@ hipError_t launch_sdd_scalars(int mode, const double* part, double* sc, double* 
                               hipStream_t s);
 template <typename T> hipError_t launch_etd_residual(const EtdArgs<T>& a, hipStream_t s);
 template <typename T> hipError_t launch_kgrad(const KGradArgs<T>& a, int ndim, hipStream_t s);
-template <typename T> hipError_t launch_kelastic(const KElasticArgs<T>& a, hipStream_t s);
 template <typename T> hipError_t launch_kelastic_table(const KElasticArgs<T>& a, T* ktab, hipStream_t s);
 // VolumeConservingLP.OnStepFinished (volumeConserving.go:31-50) on device state
 // st = {Multiplier, CurrentIntegral, IsFirstUpdate}: the field integral is the sum of the
-// partials px[0..nb), the indicator integral *ind (the zero mode of a k-space derived brick,
-// or element 0 of a real field)
-template <typename T> hipError_t launch_volcons_update(const double* px, long nb, const T* ind, double dt,
-                                                       double* st, hipStream_t s);
+// partials px[0..nb), the indicator integral the sum of cnt values `stride` apart from ind (the
+// zero mode of a k-space derived brick, the line that sums to it, or element 0 of a real field)
+template <typename T> hipError_t launch_volcons_update(const double* px, long nb, const T* ind, long cnt, long stride,
+                                                       double dt, double* st, hipStream_t s);
 // out = factor * sum_d w_d^2
 template <typename T> hipError_t launch_sqsum(const T* const* w, int nw, T factor, T* out, long n, hipStream_t s);
 template <typename T> hipError_t launch_copy(const T* src, T* dst, long n, hipStream_t s);

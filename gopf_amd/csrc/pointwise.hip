@@ -480,13 +480,19 @@ __global__ void k_etd_residual(EtdArgs<T> a) {
     }
 }
 
+// one wavefront; ind is one value, or cnt of them `stride` apart to be summed
 template <typename T>
-__global__ void k_volcons_update(const double* __restrict__ px, long nb, const T* __restrict__ ind, double dt,
-                                 double* __restrict__ st) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double fi = 0.0;
-    for (long b = 0; b < nb; ++b) fi += px[b];
-    const double ii = (double)ind[0];
+__global__ void __launch_bounds__(64) k_volcons_update(const double* __restrict__ px, long nb,
+                                                       const T* __restrict__ ind, long cnt, long stride, double dt,
+                                                       double* __restrict__ st) {
+    double fi = 0.0, ii = 0.0;
+    for (long b = threadIdx.x; b < nb; b += 64) fi += px[b];
+    for (long c = threadIdx.x; c < cnt; c += 64) ii += (double)ind[c * stride];
+    for (int o = 32; o > 0; o >>= 1) {
+        fi += __shfl_xor(fi, o, 64);
+        ii += __shfl_xor(ii, o, 64);
+    }
+    if (threadIdx.x != 0) return;
     if (st[2] != 0.0) {
         st[1] = fi;
         st[2] = 0.0;
@@ -618,15 +624,6 @@ __global__ void k_kelastic_table(KElasticArgs<T> a, T* __restrict__ ktab) {
         double f[3];
         ref_freq(a.g, kx, ky, kz, f);
         ktab[i] = (T)elastic_kernel(a.ep, f);
-    }
-}
-
-template <typename T>
-__global__ void k_kelastic(KElasticArgs<T> a) {
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < a.nk; i += (long)gridDim.x * blockDim.x) {
-        const double K = (double)a.ktab[i];
-        const cpx<T> s = a.src[i];
-        a.dst[i] = mk<T>((T)(K * (double)s.x), (T)(K * (double)s.y));
     }
 }
 
@@ -1083,8 +1080,9 @@ hipError_t launch_etd_residual(const EtdArgs<T>& a, hipStream_t s) {
     return hipGetLastError();
 }
 template <typename T>
-hipError_t launch_volcons_update(const double* px, long nb, const T* ind, double dt, double* st, hipStream_t s) {
-    hipLaunchKernelGGL(k_volcons_update<T>, dim3(1), dim3(64), 0, s, px, nb, ind, dt, st);
+hipError_t launch_volcons_update(const double* px, long nb, const T* ind, long cnt, long stride, double dt, double* st,
+                                 hipStream_t s) {
+    hipLaunchKernelGGL(k_volcons_update<T>, dim3(1), dim3(64), 0, s, px, nb, ind, cnt, stride, dt, st);
     return hipGetLastError();
 }
 template <typename T>
@@ -1095,12 +1093,6 @@ hipError_t launch_kgrad(const KGradArgs<T>& a, int ndim, hipStream_t s) {
 template <typename T>
 hipError_t launch_kelastic_table(const KElasticArgs<T>& a, T* ktab, hipStream_t s) {
     hipLaunchKernelGGL(k_kelastic_table<T>, dim3(grid_for(a.nk)), dim3(256), 0, s, a, ktab);
-    return hipGetLastError();
-}
-template <typename T>
-hipError_t launch_kelastic(const KElasticArgs<T>& a, hipStream_t s) {
-    if (!a.ktab) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_kelastic<T>, dim3(grid_for(a.nk)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 template <typename T>
@@ -1240,9 +1232,9 @@ hipError_t launch_reduce2(const double* a, long na, double ca, const double* b, 
     template hipError_t launch_etd_residual<T>(const EtdArgs<T>&, hipStream_t);                               \
     template hipError_t launch_rk4_stage<T>(const Rk4StageArgs<T>&, hipStream_t);                             \
     template hipError_t launch_stage_denoms<T>(const StageDenomArgs<T>&, hipStream_t);                        \
-    template hipError_t launch_volcons_update<T>(const double*, long, const T*, double, double*, hipStream_t); \
+    template hipError_t launch_volcons_update<T>(const double*, long, const T*, long, long, double, double*,    \
+                                                 hipStream_t);                                                \
     template hipError_t launch_kgrad<T>(const KGradArgs<T>&, int, hipStream_t);                               \
-    template hipError_t launch_kelastic<T>(const KElasticArgs<T>&, hipStream_t);                              \
     template hipError_t launch_kelastic_table<T>(const KElasticArgs<T>&, T*, hipStream_t);                    \
     template hipError_t launch_sqsum<T>(const T* const*, int, T, T*, long, hipStream_t);                      \
     template hipError_t launch_copy<T>(const T*, T*, long, hipStream_t);                                      \
