@@ -46,6 +46,7 @@
 #include "pointwise.h"
 #include "spectral.h"
 #include "spectral_mid.h"
+#include "spectral_rowpoly.h"
 
 namespace gpf {
 
@@ -604,7 +605,15 @@ private:
     void implicit_residual(const double* x, double* out);
     void implicit_jv(const double* v, double* out);
     int implicit_gmres();
-    double dev_scalar(const double* p);
+    // the residual or (npt > 0) its directional derivative along v through the middle pass
+    bool etd_mid_eligible();
+    void etd_mid(const double* x, const double* v, int npt, const double* off, const double* w, double* out);
+    std::vector<Buf<double>> etd_w_;   // weight of the explicit part in the update, per field
+    std::vector<Buf<cpx<T>>> etd_cc_;  // the residual's constant part, per field
+    // results a kernel leaves for the host: the Gram-Schmidt coefficients and norm of an Arnoldi
+    // step, |F|_max (mapped pinned memory)
+    double* nk_host_ = nullptr;
+    double* nk_map_ = nullptr;
     struct NewtonKrylov {
         int maxiter = 50;       // DefaultNonLinSolver (implicitEuler.go:221-229)
         double step = 1e-3;
@@ -617,8 +626,7 @@ private:
     std::vector<Buf<cpx<T>>> ORIG_, RP_, RES_;
     // Newton-Krylov vectors of length nf n: iterate, residual, update, perturbed point,
     // residual there, Arnoldi work vector, GMRES basis (restart + 1 vectors)
-    Buf<double> nx_, nfx_, ndx_, nxp_, nfp_, nw_, nv_, npart_, ndev_;
-    std::vector<double> nhost_;
+    Buf<double> nx_, nfx_, ndx_, nxp_, nfp_, nw_, nv_, npart_;
     // SDD (sdd.go:84-301): orientation (nf n, unit norm), its spectra, the right-hand sides at
     // the dimer's ends, the real torque, partial sums, device scalars and monitors
     void sdd_step();
@@ -841,11 +849,11 @@ Engine<T>::Engine(const Model& m, const int* dims, int ndim, double dt, const gp
             nx_.alloc(M);
             nfx_.alloc(M);
             ndx_.alloc(M);
-            nxp_.alloc(M);
-            nfp_.alloc(M);
             nw_.alloc(M);
-            npart_.alloc(krylov_blocks(M) * (kMaxKrylov + 1));
-            ndev_.alloc(4 * (kMaxKrylov + 1));
+            npart_.alloc(std::max(krylov_blocks(M), 2 * gs_blocks(M) * (kMaxKrylov + 1)));
+            HIPCHK(hipHostMalloc(reinterpret_cast<void**>(&nk_host_), (2 * (kMaxKrylov + 1) + 1) * sizeof(double),
+                                 hipHostMallocMapped));
+            HIPCHK(hipHostGetDevicePointer(reinterpret_cast<void**>(&nk_map_), nk_host_, 0));
         }
         // derived-field programs
         for (int d = 0; d < nd_; ++d) {
@@ -902,6 +910,7 @@ Engine<T>::~Engine() {
         (void)hipStreamDestroy(st_);
     }
     if (pfail_) (void)hipHostFree(pfail_);
+    if (nk_host_) (void)hipHostFree(nk_host_);
 }
 
 template <typename T>
@@ -2366,17 +2375,87 @@ void Engine<T>::general_step_rk4() {
     }
 }
 
+// The residual is linear in the spectra of the fields and of the derived fields, with weights that
+// depend on k only, where the explicit terms are of the middle pass's kinds and the derived fields
+// are dense polynomials: F(x)^ = x^ + sum_t w L^p_t B_t^(x) + cc, w and cc fixed within a step.
+// One row pass, the middle pass and the inverse rows are then the whole residual, and its finite
+// difference along v is one evaluation of the same form with v for x and the stencil's sum of the
+// pointwise sources for B_t (the constant terms drop out, the stencil's weights summing to 0).
 template <typename T>
-double Engine<T>::dev_scalar(const double* p) {
-    double v = 0.0;
-    HIPCHK(hipMemcpyAsync(&v, p, sizeof(double), hipMemcpyDeviceToHost, st_));
-    HIPCHK(hipStreamSynchronize(st_));
-    return v;
+bool Engine<T>::etd_mid_eligible() {
+    if (sizeof(T) != 8 || !row_sync_ || nf_ + nd_ > kMaxArr || !mid_eligible()) return false;
+    for (int i = 0; i < nf_; ++i)
+        if (eqs_[i].terms.size() + 1 > (size_t)kMidTerms) return false;
+    return true;
+}
+
+template <typename T>
+void Engine<T>::etd_mid(const double* x, const double* v, int npt, const double* off, const double* w, double* out) {
+    if constexpr (std::is_same<T, double>::value) {
+        const long n = g_.n;
+        RowPolyArgs r;
+        r.tw = tw(g_.nx);
+        r.nf = nf_;
+        r.nd = nd_;
+        r.x = x;
+        r.v = v;
+        r.n = n;
+        r.npt = npt;
+        for (int k = 0; k < npt; ++k) {
+            r.off[k] = off[k];
+            r.w[k] = w[k];
+        }
+        std::vector<cpx<T>*> lines;
+        for (int b = 0; b < nf_ + nd_; ++b) {
+            r.out[b] = K_[b].get();
+            lines.push_back(K_[b].get());
+        }
+        for (int d = 0; d < nd_; ++d) std::memcpy(r.dc[d], dargs_[d].dc, sizeof(r.dc[d]));
+        r.nmain = g_.nmain;
+        r.rows = g_.rows;
+        r.nx = g_.nx;
+        r.TW = spread_tw(choose_tw(g_.nx, 1, sizeof(cpx<T>), 1, 1), g_.rows);
+        HIPCHK(launch_rows_poly(r, st_));
+        if (g_.ndim == 3) pencils(lines, {}, 1, -1);
+        MidArgs<T> a = mid_args(kMidResidual);
+        a.nf = nf_;
+        std::vector<const cpx<T>*> in;
+        std::vector<T*> o;
+        for (int i = 0; i < nf_; ++i) {
+            MidField<T>& f = a.f[i];
+            mid_terms(i, a, f, 1);
+            f.t[0] = MidTerm<T>();
+            f.t[0].b = K_[i].get();
+            f.t[0].line = 1;
+            int keep = 1;
+            for (int q = 1; q < f.nterm; ++q) {
+                MidTerm<T> t = f.t[q];
+                for (int j = 0; j < nf_; ++j) t.line |= (t.b == K_[j].get()) ? 1 : 0;
+                if (npt > 0 && !t.line) continue;  // constant along v
+                f.t[keep++] = t;
+            }
+            f.nterm = keep;
+            f.s64 = etd_w_[i].get();
+            f.cc = npt > 0 ? nullptr : etd_cc_[i].get();
+            // the residual leaves the fields' spectra for the next step where no other line of
+            // the launch reads them
+            f.kn = (npt == 0 && !mid_self_) ? K_[i].get() : nullptr;
+            f.out = kscratch(i);
+            in.push_back(nullptr);
+            o.push_back(out + i * n);
+        }
+        launch_mid_pass(a);
+        c2r(in, o, T(1) / (T)n, nullptr, false);
+    }
 }
 
 template <typename T>
 void Engine<T>::implicit_residual(const double* x, double* out) {
     if constexpr (std::is_same<T, double>::value) {
+        if (etd_mid_eligible()) {
+            etd_mid(x, nullptr, 0, nullptr, nullptr, out);
+            return;
+        }
         const long n = g_.n;
         std::vector<const T*> in;
         std::vector<cpx<T>*> ko;
@@ -2457,6 +2536,24 @@ template <typename T>
 void Engine<T>::implicit_jv(const double* v, double* out) {
     const long M = (long)nf_ * g_.n;
     const double h = nk_.step;
+    if (etd_mid_eligible()) {
+        double off[8] = {0.0, h}, w[8] = {-1.0 / h, 1.0 / h};
+        int npt = 2;
+        if (nk_.stencil != 1) {
+            const FdStencil& fd = kFdStencils[nk_.stencil / 2 - 1];
+            npt = fd.n;
+            for (int k = 0; k < npt; ++k) {
+                off[k] = fd.off[k] * h;
+                w[k] = fd.w[k] / h;
+            }
+        }
+        etd_mid(nx_.get(), v, npt, off, w, out);
+        return;
+    }
+    if (!nxp_.get()) {
+        nxp_.alloc(M);
+        nfp_.alloc(M);
+    }
     if (nk_.stencil == 1) {
         HIPCHK(launch_axpby(1.0, nx_.get(), h, v, nxp_.get(), M, st_));
         implicit_residual(nxp_.get(), nfp_.get());
@@ -2476,23 +2573,26 @@ template <typename T>
 int Engine<T>::implicit_gmres() {
     const long M = (long)nf_ * g_.n;
     const int m = nk_.restart;
-    const long nb = krylov_blocks(M);
     constexpr int kStride = kMaxKrylov + 1;
     double* V = nv_.get();
-    double* dev = ndev_.get();  // [0, kStride) CGS pass 1, [kStride, 2 kStride) pass 2, [2 kStride] |w|^2,
-                                // [3 kStride, 4 kStride) solution coefficients
-    HIPCHK(hipMemsetAsync(ndx_.get(), 0, M * sizeof(double), st_));
-    HIPCHK(launch_axpby(0.0, nullptr, -1.0, nfx_.get(), nw_.get(), M, st_));
-    HIPCHK(launch_multidot(nw_.get(), M, 1, nw_.get(), M, npart_.get(), st_));
-    HIPCHK(launch_reduce_rows(npart_.get(), 1, nb, dev + 2 * kStride, st_));
-    HIPCHK(launch_normalize(nw_.get(), dev + 2 * kStride, V, M, st_));
-    double beta = std::sqrt(std::max(dev_scalar(dev + 2 * kStride), 0.0));
-    if (!(beta > 0.0) || !std::isfinite(beta)) return 0;
+    // two sets of partial sums (a sweep reads one and writes the other); the host reads from
+    // nk_host_: [0, kStride) the coefficients of pass 1, [kStride, 2 kStride) pass 2,
+    // [2 kStride] |w|^2
+    double* pa = npart_.get();
+    double* pb = pa + gs_blocks(M) * kStride;
+    const double* host = nk_host_;
+    HIPCHK(launch_gs_dots(nfx_.get(), M, 1, nfx_.get(), M, pa, st_));
+    HIPCHK(launch_gs_normalize(pa, nfx_.get(), -1.0, V, M, nk_map_ + 2 * kStride, st_));
+    HIPCHK(hipStreamSynchronize(st_));
+    double beta = std::sqrt(std::max(host[2 * kStride], 0.0));
+    if (!(beta > 0.0) || !std::isfinite(beta)) {
+        HIPCHK(hipMemsetAsync(ndx_.get(), 0, M * sizeof(double), st_));
+        return 0;
+    }
     // the linear model needs no residual far below the Newton tolerance (max norm <= 2-norm)
     const double target = std::max(1e-10 * beta, 0.1 * nk_.tol);
     std::vector<double> H((size_t)(m + 1) * m), Hu((size_t)(m + 1) * m), cs(m), sn(m), g(m + 1), y(m + 1);
     auto at = [m](std::vector<double>& A, int i, int j) -> double& { return A[(size_t)i * m + j]; };
-    nhost_.assign(2 * kStride + 1, 0.0);
     int total = 0;
     const int max_cycles = 10;
     for (int cycle = 0; cycle < max_cycles; ++cycle) {
@@ -2506,20 +2606,13 @@ int Engine<T>::implicit_gmres() {
             double* w = nw_.get();
             implicit_jv(V + (long)j * M, w);
             // classical Gram-Schmidt, twice
-            HIPCHK(launch_multidot(V, M, j + 1, w, M, npart_.get(), st_));
-            HIPCHK(launch_reduce_rows(npart_.get(), j + 1, nb, dev, st_));
-            HIPCHK(launch_combine(V, M, j + 1, dev, -1.0, w, M, st_));
-            HIPCHK(launch_multidot(V, M, j + 1, w, M, npart_.get(), st_));
-            HIPCHK(launch_reduce_rows(npart_.get(), j + 1, nb, dev + kStride, st_));
-            HIPCHK(launch_combine(V, M, j + 1, dev + kStride, -1.0, w, M, st_));
-            HIPCHK(launch_multidot(w, M, 1, w, M, npart_.get(), st_));
-            HIPCHK(launch_reduce_rows(npart_.get(), 1, nb, dev + 2 * kStride, st_));
-            HIPCHK(launch_normalize(w, dev + 2 * kStride, V + (long)(j + 1) * M, M, st_));
-            HIPCHK(hipMemcpyAsync(nhost_.data(), dev, (2 * kStride + 1) * sizeof(double), hipMemcpyDeviceToHost,
-                                  st_));
+            HIPCHK(launch_gs_dots(V, M, j + 1, w, M, pa, st_));
+            HIPCHK(launch_gs_sweep(V, M, j + 1, pa, w, M, true, pb, nk_map_, st_));
+            HIPCHK(launch_gs_sweep(V, M, j + 1, pb, w, M, false, pa, nk_map_ + kStride, st_));
+            HIPCHK(launch_gs_normalize(pa, w, 1.0, V + (long)(j + 1) * M, M, nk_map_ + 2 * kStride, st_));
             HIPCHK(hipStreamSynchronize(st_));
-            for (int i = 0; i <= j; ++i) at(Hu, i, j) = at(H, i, j) = nhost_[i] + nhost_[kStride + i];
-            const double hn = std::sqrt(std::max(nhost_[2 * kStride], 0.0));
+            for (int i = 0; i <= j; ++i) at(Hu, i, j) = at(H, i, j) = host[i] + host[kStride + i];
+            const double hn = std::sqrt(std::max(host[2 * kStride], 0.0));
             at(Hu, j + 1, j) = at(H, j + 1, j) = hn;
             // Givens rotations of the least-squares problem min |g - H y|
             for (int i = 0; i < j; ++i) {
@@ -2537,7 +2630,10 @@ int Engine<T>::implicit_gmres() {
             g[j] = cs[j] * g[j];
             ++total;
             jend = j + 1;
-            if (!std::isfinite(g[j + 1])) return total;
+            if (!std::isfinite(g[j + 1])) {
+                if (cycle == 0) HIPCHK(hipMemsetAsync(ndx_.get(), 0, M * sizeof(double), st_));
+                return total;
+            }
             if (std::fabs(g[j + 1]) <= target || !(hn > 1e-14 * beta)) {
                 done = true;
                 break;
@@ -2549,22 +2645,20 @@ int Engine<T>::implicit_gmres() {
             for (int k = i + 1; k < jend; ++k) t -= at(H, i, k) * y[k];
             y[i] = (at(H, i, i) != 0.0) ? t / at(H, i, i) : 0.0;
         }
-        HIPCHK(hipMemcpyAsync(dev + 3 * kStride, y.data(), jend * sizeof(double), hipMemcpyHostToDevice, st_));
-        HIPCHK(launch_combine(V, M, jend, dev + 3 * kStride, 1.0, ndx_.get(), M, st_));
-        HIPCHK(hipStreamSynchronize(st_));
+        KrylovCoefs yc{};
+        for (int i = 0; i < jend; ++i) yc.v[i] = y[i];
+        HIPCHK(launch_expand(V, M, jend, yc, cycle == 0 ? nullptr : ndx_.get(), ndx_.get(), M, st_));
         if (done || cycle + 1 == max_cycles) break;
         // restart from the Arnoldi residual r = V_{m+1} (beta e1 - Hu y)
-        std::vector<double> z(jend + 1, 0.0);
-        z[0] = beta;
+        KrylovCoefs z{};
+        z.v[0] = beta;
         for (int i = 0; i <= jend; ++i)
-            for (int k = 0; k < jend; ++k) z[i] -= at(Hu, i, k) * y[k];
-        HIPCHK(hipMemcpyAsync(dev + 3 * kStride, z.data(), (jend + 1) * sizeof(double), hipMemcpyHostToDevice, st_));
-        HIPCHK(hipMemsetAsync(nw_.get(), 0, M * sizeof(double), st_));
-        HIPCHK(launch_combine(V, M, jend + 1, dev + 3 * kStride, 1.0, nw_.get(), M, st_));
-        HIPCHK(launch_multidot(nw_.get(), M, 1, nw_.get(), M, npart_.get(), st_));
-        HIPCHK(launch_reduce_rows(npart_.get(), 1, nb, dev + 2 * kStride, st_));
-        HIPCHK(launch_normalize(nw_.get(), dev + 2 * kStride, V, M, st_));
-        beta = std::sqrt(std::max(dev_scalar(dev + 2 * kStride), 0.0));
+            for (int k = 0; k < jend; ++k) z.v[i] -= at(Hu, i, k) * y[k];
+        HIPCHK(launch_expand(V, M, jend + 1, z, nullptr, nw_.get(), M, st_));
+        HIPCHK(launch_gs_dots(nw_.get(), M, 1, nw_.get(), M, pa, st_));
+        HIPCHK(launch_gs_normalize(pa, nw_.get(), 1.0, V, M, nk_map_ + 2 * kStride, st_));
+        HIPCHK(hipStreamSynchronize(st_));
+        beta = std::sqrt(std::max(host[2 * kStride], 0.0));
         if (!(beta > target) || !std::isfinite(beta)) break;
     }
     return total;
@@ -2585,6 +2679,25 @@ void Engine<T>::implicit_step() {
         rhs_update(i, RP_[i].get(), nullptr, 0.0, 1.0, 0.0, false, nullptr);
         HIPCHK(hipMemcpyAsync(ORIG_[i].get(), K_[i].get(), kb, hipMemcpyDeviceToDevice, st_));
     }
+    const bool mid = etd_mid_eligible();
+    for (int i = 0; i < nf_ && mid; ++i) {
+        while ((int)etd_w_.size() <= i) {
+            etd_w_.emplace_back(g_.nk);
+            etd_cc_.emplace_back(g_.nk);
+        }
+        EtdArgs<T> a;
+        a.dst = etd_cc_[i].get();
+        a.orig = ORIG_[i].get();
+        a.rprev = RP_[i].get();
+        a.denom = eqs_[i].denom;
+        a.sv = eqs_[i].sv;
+        a.hs = eqs_[i].hs;
+        a.dt = dt_;
+        a.g = g_.kg;
+        a.nmain = g_.nmain;
+        a.nk = g_.nk;
+        HIPCHK(launch_etd_tables<T>(a, etd_w_[i].get(), st_));
+    }
     // explicit Euler step as the initial guess (implicitEuler.go:182-190; euler.go:32-44 with
     // the stepper's filter), from the right-hand side just formed
     std::vector<const cpx<T>*> in;
@@ -2601,11 +2714,11 @@ void Engine<T>::implicit_step() {
     nk_newton_ = 0;
     nk_krylov_ = 0;
     nk_conv_ = 0;
-    double* dev = ndev_.get();
     for (int it = 0; it < nk_.maxiter; ++it) {
         implicit_residual(nx_.get(), nfx_.get());
-        HIPCHK(launch_absmax(nfx_.get(), M, npart_.get(), dev, st_));
-        nk_res_ = dev_scalar(dev);
+        HIPCHK(launch_absmax(nfx_.get(), M, npart_.get(), nk_map_, st_));
+        HIPCHK(hipStreamSynchronize(st_));
+        nk_res_ = nk_host_[0];
         if (nk_res_ < nk_.tol) {
             nk_conv_ = 1;
             break;
@@ -2617,10 +2730,11 @@ void Engine<T>::implicit_step() {
     }
     if (!nk_conv_) std::fprintf(stderr, "Warning: Iterative solver did not converge\n");
     // the fields take the solution (implicitEuler.go:205); after a converged check the
-    // k-space bricks of the fields are FFT(x) already
+    // k-space bricks of the fields are FFT(x) already (the middle pass leaves them unless an
+    // equation reads a field's spectrum)
     for (int i = 0; i < nf_; ++i)
         HIPCHK(hipMemcpyAsync(F_[i].get(), nx_.get() + i * n, n * sizeof(T), hipMemcpyDeviceToDevice, st_));
-    kvalid_ = nk_conv_ != 0;
+    kvalid_ = nk_conv_ != 0 && !(mid && mid_self_);
 }
 
 template <typename T>

@@ -319,6 +319,9 @@ hipError_t launch_sdd_orient(double* v, const double* tau, long n, double c, dou
 hipError_t launch_sdd_scalars(int mode, const double* part, double* sc, double* mon, double a0, double a1,
                               hipStream_t s);
 template <typename T> hipError_t launch_etd_residual(const EtdArgs<T>& a, hipStream_t s);
+// w[k] = the weight of R in the residual, dst = its part that does not depend on the iterate
+// (a.orig, a.rprev, the denominator; terms unused)
+template <typename T> hipError_t launch_etd_tables(const EtdArgs<T>& a, double* w, hipStream_t s);
 template <typename T> hipError_t launch_kgrad(const KGradArgs<T>& a, int ndim, hipStream_t s);
 template <typename T> hipError_t launch_kelastic_table(const KElasticArgs<T>& a, T* ktab, hipStream_t s);
 // VolumeConservingLP.OnStepFinished (volumeConserving.go:31-50) on device state

@@ -480,6 +480,34 @@ __global__ void k_etd_residual(EtdArgs<T> a) {
     }
 }
 
+// The residual's fixed parts within a step (spectral_mid.h, kMidResidual): with I = w_r R + w_p P the
+// integral above, w = -w_r and dst = -(orig e^{D dt} + w_p P); conjugate-averaged where the update is
+template <typename T>
+__global__ void k_etd_tables(EtdArgs<T> a, double* __restrict__ w) {
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < a.nk; i += (long)gridDim.x * blockDim.x) {
+        int kx, ky, kz;
+        kcoords(a.g, i, a.nmain, kx, ky, kz);
+        double f[3];
+        ref_freq(a.g, kx, ky, kz, f);
+        const double f2 = f[0] * f[0] + f[1] * f[1] + f[2] * f[2];
+        const double L = -(4.0 * kPi * kPi) * f2;
+        // the weights are the integrals of a unit right-hand side and of a unit previous one
+        double e, wr, wp;
+        etd_update(denominator(a.denom, a.sv, a.hs, a.g.ndim, f, L, f2), a.dt, 1.0, 0.0, 0.0, 1.0, e, wr, wp);
+        if (asym_row(a.hs, a.g.ndim, f)) {
+            double fc[3], ec, wrc, wpc;
+            conj_freq(a.g.ndim, f, fc);
+            etd_update(denominator(a.denom, a.sv, a.hs, a.g.ndim, fc, L, f2), a.dt, 1.0, 0.0, 0.0, 1.0, ec, wrc, wpc);
+            e = 0.5 * (e + ec);
+            wr = 0.5 * (wr + wrc);
+            wp = 0.5 * (wp + wpc);
+        }
+        const cpx<T> o = a.orig[i], p = a.rprev[i];
+        w[i] = -wr;
+        a.dst[i] = mk<T>((T)(-((double)o.x * e + wp * (double)p.x)), (T)(-((double)o.y * e + wp * (double)p.y)));
+    }
+}
+
 // one wavefront; ind is one value, or cnt of them `stride` apart to be summed
 template <typename T>
 __global__ void __launch_bounds__(64) k_volcons_update(const double* __restrict__ px, long nb,
@@ -1075,6 +1103,11 @@ hipError_t launch_stage_denoms(const StageDenomArgs<T>& a, hipStream_t s) {
     return hipGetLastError();
 }
 template <typename T>
+hipError_t launch_etd_tables(const EtdArgs<T>& a, double* w, hipStream_t s) {
+    hipLaunchKernelGGL(k_etd_tables<T>, dim3(grid_for(a.nk)), dim3(256), 0, s, a, w);
+    return hipGetLastError();
+}
+template <typename T>
 hipError_t launch_etd_residual(const EtdArgs<T>& a, hipStream_t s) {
     hipLaunchKernelGGL(k_etd_residual<T>, dim3(grid_for(a.nk)), dim3(256), 0, s, a);
     return hipGetLastError();
@@ -1230,6 +1263,7 @@ hipError_t launch_reduce2(const double* a, long na, double ca, const double* b, 
     template hipError_t launch_derived<T>(const DerivedArgs<T>&, hipStream_t);                                \
     template hipError_t launch_kupdate<T>(const KUpdateArgs<T>&, hipStream_t);                                \
     template hipError_t launch_etd_residual<T>(const EtdArgs<T>&, hipStream_t);                               \
+    template hipError_t launch_etd_tables<T>(const EtdArgs<T>&, double*, hipStream_t);                        \
     template hipError_t launch_rk4_stage<T>(const Rk4StageArgs<T>&, hipStream_t);                             \
     template hipError_t launch_stage_denoms<T>(const StageDenomArgs<T>&, hipStream_t);                        \
     template hipError_t launch_volcons_update<T>(const double*, long, const T*, long, long, double, double*,    \
