@@ -253,25 +253,47 @@ static bool tw_fits(int n, int tw, size_t elem, int variant = 0) {
     return tw * T <= kMaxBlockThreads && lds <= 160 * 1024;
 }
 
-static int choose_tw(int n, int narr, size_t elem, int min_tw, int variant = 0, int threads = 256) {
-    const int T = fft_threads_per_line(n, variant);
+// lines per block of the stand-alone transforms: about 256 threads, at least min_tw lines
+static int choose_tw(int n, size_t elem, int min_tw) {
+    const int T = fft_threads_per_line(n, 0);
     int tw = 1;
-    while (tw * 2 * T <= threads) tw *= 2;  // lines per block: a power of two
+    while (tw * 2 * T <= 256) tw *= 2;  // lines per block: a power of two
     if (tw > 64) tw = 64;
     while (tw < min_tw && tw * 2 * T <= 256) tw *= 2;
     while (tw * T > kMaxBlockThreads && tw > 1) tw /= 2;
-    (void)narr;
     while (tw > 1 && (size_t)(n + n / 16 + 1) * (tw + 1) * elem > 80 * 1024) tw /= 2;
     return tw;
 }
 
-// lines per block of a general-path pass over `lines` lines: a small grid's pass is
-// latency-bound, so fewer lines per block spread it over at least kSpreadBlocks workgroups
-// (at 128^2 the row transform ran on 4 workgroups); large grids keep tw
-constexpr long kSpreadBlocks = 256;
-static int spread_tw(int tw, long lines, int min_tw = 1) {
-    while (tw > min_tw && (lines + tw - 1) / tw < kSpreadBlocks) tw /= 2;
-    return tw;
+// Lines per block of a pass whose launch layout is not tuned: the power of two with the least
+// work per CU, max(tw, 64 / T) lines per block times the blocks per CU (at least one).  A block of
+// fewer than 64 threads leaves a wavefront part empty; strided passes of one or two lines per
+// block use 8 to 32 bytes of a cache line at a time.  Blocks of one wavefront have no barrier
+// between wavefronts, so ties go to the smallest block of at least 64 threads while the lines
+// are shorter than that and the launch is short (rows 5000 wavefronts, strided 4000: 128^3 FP32
+// rows, 256 blocks of 256 threads against 1024 of 64, 40.0 -> 33.9 us a step; 48^3 and 96^3 25.5 ->
+// 19.3 and 30.8 -> 28.6), otherwise to the largest (256^3 FP32 122.9 -> 121.4, 2048^2 FP32 rows
+// 62.1 -> 56.6, 512^2 FP32 update 13.7 -> 12.6).  At most 256 threads, and 128 for the strided FP64
+// passes, whose LDS would leave two blocks per CU (192^3 129 -> 123 us a step, 256^3 234 -> 230),
+// but two lines of a long transform.  blocks(tw): the launch's blocks.
+template <typename F>
+static int fit_tw(int n, size_t elem, int variant, bool strided, long lines, F&& blocks, int min_threads = 0) {
+    const int T = fft_threads_per_line(n, variant);
+    const int most = std::max((strided && elem == 16) ? 128 : 256, std::min(2 * T, kMaxBlockThreads));
+    const bool small = T < 64 && (double)lines * T <= (strided ? 4096.0 : 5120.0) * 64.0;
+    int best = 1;
+    double bc = 1e300;
+    for (int tw = 64; tw >= 1; tw /= 2) {
+        if (tw > 1 && (tw * T > most || (size_t)(n + n / 16 + 1) * (tw + 1) * elem > 80 * 1024)) continue;
+        if (tw * T < min_threads && bc < 1e300) continue;
+        const double pen = !strided || tw >= 8 ? 1.0 : tw == 4 ? 1.05 : tw == 2 ? 1.2 : 2.4;
+        const double c = std::max((double)blocks(tw) / 256.0, 1.0) * std::max((double)tw, 64.0 / T) * pen;
+        if (c < 0.97 * bc || (small && tw * T >= 64 && c <= 1.03 * bc)) {
+            bc = std::min(c, bc);
+            best = tw;
+        }
+    }
+    return best;
 }
 
 static Seg seg_y_main(const Geometry& g) {
@@ -552,8 +574,13 @@ private:
     long pnr_ = 0, pnu_ = 0;  // block counts of the plan's row and update passes
     Buf<unsigned> pbar_;
     Buf<double> ppa_bulk_, ppa_mass_, ppc_eg_;
-    Buf<cpx<T>> ptab_;  // the update pass's multipliers of every k-point
-    Buf<double> pm0_;   // m1(0), m2(0)
+    // the update pass's multipliers of every k-point, tabulated once (they are the same every
+    // step), and m1(0), m2(0)
+    Buf<cpx<T>> ptab_;
+    Buf<double> pm0_;
+    bool ptab_ok_ = false;
+    void update_table(PencilUpdateArgs<T>& u);
+    bool table_pays() const;
     int* pfail_ = nullptr;      // mapped host flag set by a failed device-wide barrier
     int* pfail_dev_ = nullptr;
     PersistLaunch<T> pl_;
@@ -575,6 +602,11 @@ private:
     int upd_axis() const { return (g_.ndim == 3) ? upd_axis_ : 1; }
     int other_axis() const { return upd_axis() == 2 ? 1 : 2; }
     int axis_len(int axis) const { return axis == 2 ? g_.nz : g_.ny; }
+    // lines per block of an untuned row pass over `lines` transform lines
+    int rows_tw(long lines, int variant = 0, int min_threads = 0) const {
+        return fit_tw(g_.nx, sizeof(cpx<T>), variant, false, lines, [&](int tw) { return (lines + tw - 1) / tw; },
+                      min_threads);
+    }
     // general path
     void general_step_euler();
     void general_step_rk4();
@@ -733,6 +765,15 @@ Engine<T>::Engine(const Model& m, const int* dims, int ndim, double dt, const gp
         W_.alloc(g_.nk);
         mean_.alloc(1);
         split_mean_ = (sizeof(T) == 4);
+        // untuned update axis: y, whose arrays are then read within a plane (us per step, z and y:
+        // 256^3 FP64 262 and 234, 128^3 55.6 and 44.1, FP32 128^3 38.0 and 33.9, 160^3 63.0 and
+        // 59.4, 192^3 69.2 and 67.6), but for large FP32 grids, where both take the same time
+        // (256^3 119.4)
+        upd_axis_ = (sizeof(T) == 8 || table_pays()) ? 1 : 2;
+        // untuned row pass: the low-register schedule where the plain one has at most 512
+        // wavefronts, so that a row's chain is shorter (256^2 13.6 -> 13.0 us a step, 1024^2 FP32
+        // 25.7 -> 24.4; 256^3 FP32 the other way, 119 -> 124)
+        rows_var_ = (g_.rows + 1) / 2 * (long)fft_threads_per_line(g_.nx, 0) <= 512 * 64 ? 1 : 0;
         pass_names_ = {"rows_fused", "pencils_fwd", "pencil_update", "pencils_inv"};
     } else {
         // compile every equation for the general path
@@ -991,10 +1032,8 @@ void Engine<T>::pencils(const std::vector<cpx<T>*>& dst, const std::vector<const
         a.seg[0] = (axis == 1) ? seg_y_main(g_) : seg_z_main(g_);
         a.seg[1] = (axis == 1) ? seg_y_nyq(g_) : seg_z_nyq(g_);
         a.nseg = 2;
-        // about 128 threads per block: at 192^3 (C4) 8 lines per block beat 16 by 1 % (FP32)
-        // and 3 % (FP64) per step
-        a.TW = spread_tw(choose_tw(n, a.narr, sizeof(cpx<T>), 8, 0, 128),
-                         (long)a.seg[0].na * a.seg[0].nb + (long)a.seg[1].na * a.seg[1].nb);
+        a.TW = fit_tw(n, sizeof(cpx<T>), 0, true, a.narr * pencil_blocks(a.seg, a.nseg, 1, nullptr),
+                      [&](int tw) { return a.narr * pencil_blocks(a.seg, a.nseg, tw, nullptr); });
         for (int q = 0; q < a.narr; ++q) {
             a.arr[q][0] = dst[q0 + q];
             a.arr[q][1] = dst[q0 + q] + g_.nmain;
@@ -1029,7 +1068,7 @@ void Engine<T>::r2c(const std::vector<const T*>& in, const std::vector<cpx<T>*>&
         }
         a.rows = g_.rows;
         a.nx = g_.nx;
-        a.TW = spread_tw(choose_tw(g_.nx, (a.narr + 1) / 2, sizeof(cpx<T>), 1), g_.rows);
+        a.TW = rows_tw(g_.rows);
         a.in_scale = in_scale;
         HIPCHK(launch_rows_r2c<T>(a, st_));
     }
@@ -1065,7 +1104,7 @@ void Engine<T>::c2r(const std::vector<const cpx<T>*>& in, const std::vector<T*>&
         }
         a.rows = g_.rows;
         a.nx = g_.nx;
-        a.TW = spread_tw(choose_tw(g_.nx, (na + 1) / 2, sizeof(cpx<T>), 1), g_.rows);
+        a.TW = rows_tw(g_.rows);
         a.scale = scale;
         a.add_mean = (q0 == 0) ? add_mean : nullptr;
         HIPCHK(launch_rows_c2r<T>(a, st_));
@@ -1293,9 +1332,8 @@ RowFusedArgs<T> Engine<T>::rows_args(cpx<T>* W, double* mean, int tw, int var) {
     ra.g_nyq = W + g_.nmain;
     ra.rows = g_.rows;
     ra.nx = g_.nx;
-    // untuned: spread over more workgroups on small grids, down to the autotuner's smallest
-    // candidate (4 lines per block)
-    ra.TW = tw > 0 ? tw : spread_tw(choose_tw(g_.nx, 1, sizeof(cpx<T>), 1, var), (g_.rows + 1) / 2, 4);
+    // (the monitor folds the series slot into row blocks of at least 64 threads)
+    ra.TW = tw > 0 ? tw : rows_tw((g_.rows + 1) / 2, var, mon_ ? 64 : 0);
     ra.variant = var;
     ra.c_out = c_out_;
     ra.npoly = (int)fp_.gpoly.size();
@@ -1319,8 +1357,8 @@ PencilUpdateArgs<T> Engine<T>::update_args(cpx<T>* S, cpx<T>* W, double* mean, i
     u.p.seg[1] = (axis == 2) ? seg_z_nyq(g_) : seg_y_nyq(g_);
     u.p.nseg = 2;
     u.p.TW = tw > 0 ? tw
-                    : spread_tw(choose_tw(nu, u.p.narr, sizeof(cpx<T>), 8, 1),
-                                (long)u.p.seg[0].na * u.p.seg[0].nb + (long)u.p.seg[1].na * u.p.seg[1].nb, 4);
+                    : fit_tw(nu, sizeof(cpx<T>), 1, true, pencil_blocks(u.p.seg, u.p.nseg, 1, nullptr),
+                             [&](int t) { return pencil_blocks(u.p.seg, u.p.nseg, t, nullptr); });
     u.g = g_.kg;
     u.dt = dt_;
     u.scale = 1.0 / (double)g_.n;
@@ -1331,7 +1369,35 @@ PencilUpdateArgs<T> Engine<T>::update_args(cpx<T>* S, cpx<T>* W, double* mean, i
     u.filter = has_filter_ ? filter_.get() : nullptr;
     u.mean = split_mean_ ? mean : nullptr;
     make_dense(u);
+    if (table_pays()) update_table(u);
     return u;
+}
+
+// Reading the multipliers costs the update pass a fifth array and saves their FP64 arithmetic (a
+// polynomial and a division per k-point) and the registers it holds.  It pays while the arrays stay
+// in the caches: us per step without and with the table, 400 x 250 FP64 20.0 and 16.4, 512^2 FP32
+// 15.0 and 12.6, 96^3 FP64 38.7 and 36.3, 160^3 FP64 104 and 92 (33 MB a spectrum), 192^3 FP32 70.0
+// and 67.6; but 192^3 FP64 (57 MB) 117.7 and 118.0, 256^3 FP32 119.5 and 125.  In 2D, whose strided
+// lines use a part of each cache line, 2000 x 1000 FP32 (8 MB) 39.4 and 36.2 but 2048^2 FP32
+// (17 MB) 60.0 and 62.1.
+template <typename T>
+bool Engine<T>::table_pays() const {
+    return (size_t)g_.nk * sizeof(cpx<T>) <= (size_t)(g_.ndim == 3 ? 40 : 12) << 20;
+}
+
+// fills the table at its first use and lets u read it; never within a graph capture, which a step's
+// preparation (prepare_fused) precedes
+template <typename T>
+void Engine<T>::update_table(PencilUpdateArgs<T>& u) {
+    if (!ptab_.get()) ptab_.alloc(g_.nk);
+    if (!pm0_.get()) pm0_.alloc(2);
+    if (!ptab_ok_) {
+        HIPCHK(launch_update_mult_table<T>(u, g_.ndim == 3 ? upd_axis() : 1, g_.nmain, g_.nk, ptab_.get(), pm0_.get(), st_));
+        ptab_ok_ = true;
+    }
+    u.mtab[0] = ptab_.get();
+    u.mtab[1] = ptab_.get() + g_.nmain;
+    u.m0 = pm0_.get();
 }
 
 // W <- S inverse-transformed along the update axis: the row-pass input of the next step
@@ -1350,8 +1416,8 @@ void Engine<T>::pencils_tw(const std::vector<cpx<T>*>& dst, int axis, int dir, i
     a.seg[1] = (axis == 1) ? seg_y_nyq(g_) : seg_z_nyq(g_);
     a.nseg = 2;
     a.TW = tw > 0 ? tw
-                  : spread_tw(choose_tw(n, a.narr, sizeof(cpx<T>), 8, var),
-                              (long)a.seg[0].na * a.seg[0].nb + (long)a.seg[1].na * a.seg[1].nb, 4);
+                  : fit_tw(n, sizeof(cpx<T>), var, true, a.narr * pencil_blocks(a.seg, a.nseg, 1, nullptr),
+                           [&](int t) { return a.narr * pencil_blocks(a.seg, a.nseg, t, nullptr); });
     a.lpt = lpt;
     a.variant = var;
     for (int q = 0; q < a.narr; ++q) {
@@ -1464,7 +1530,7 @@ void Engine<T>::set_filter(const double* table) {
     if (table && stepper_ == GPF_SDD) throw Error(GPF_EINVAL, "SDD: Does not support modal filters");
     HIPCHK(hipStreamSynchronize(st_));
     drop_graph();
-    stab_ok_ = etab_ok_ = false;
+    stab_ok_ = etab_ok_ = ptab_ok_ = false;
     if (!table) {
         has_filter_ = false;
         return;
@@ -1529,6 +1595,7 @@ void Engine<T>::drop_graph() {
 
 template <typename T>
 void Engine<T>::prepare_fused(long upcoming) {
+    if (!ptab_ok_ && table_pays()) (void)update_args(S_.get(), W_.get(), mean_.get(), tw_pu_);
     if (!mon_) return;
     const long nblk_a = rows_fused_blocks(g_.rows, rows_args(W_.get(), mean_.get(), tw_rows_, rows_var_).TW);
     PencilUpdateArgs<T> u = update_args(S_.get(), W_.get(), mean_.get(), tw_pu_);
@@ -1772,13 +1839,7 @@ void Engine<T>::build_persist() {
     const long nr = rows_fused_blocks(g_.rows, tw);
     const long nu = pencil_blocks(u.p.seg, u.p.nseg, tw, &tiles0);
     u.p.tiles0 = tiles0;
-    // the multipliers are the same every step: tabulated once, read with the lines
-    if (!ptab_.get()) ptab_.alloc(g_.nk);
-    if (!pm0_.get()) pm0_.alloc(2);
-    u.mtab[0] = ptab_.get();
-    u.mtab[1] = ptab_.get() + g_.nmain;
-    u.m0 = pm0_.get();
-    HIPCHK(launch_update_mult_table<T>(u, st_));
+    update_table(u);
     P.rows_pass = (fp_.has_src || mon_) ? 1 : 0;
     P.nblk_rows = (int)nr;
     P.nblk_upd = (int)nu;
@@ -2011,7 +2072,7 @@ void Engine<T>::eval_elastic() {
         r.dnyq[0] = Tel_[e].get() + g_.nmain;
         r.rows = g_.rows;
         r.nx = g_.nx;
-        r.TW = spread_tw(choose_tw(g_.nx, 1, sizeof(cpx<T>), 1), g_.rows);
+        r.TW = rows_tw(g_.rows);
         HIPCHK(launch_rows_sync<T>(r, st_));
         pencils({Tel_[e].get()}, {}, 1, -1);
         if (g_.ndim == 3) pencils({Tel_[e].get()}, {}, 2, -1);
@@ -2117,8 +2178,8 @@ MidArgs<T> Engine<T>::mid_args(int op) {
     a.p.seg[0] = (axis == 2) ? seg_z_main(g_) : seg_y_main(g_);
     a.p.seg[1] = (axis == 2) ? seg_z_nyq(g_) : seg_y_nyq(g_);
     a.p.nseg = 2;
-    a.p.TW = spread_tw(choose_tw(n, 1, sizeof(cpx<T>), 8, 1, 128),
-                       (long)a.p.seg[0].na * a.p.seg[0].nb + (long)a.p.seg[1].na * a.p.seg[1].nb);
+    a.p.TW = fit_tw(n, sizeof(cpx<T>), 1, true, nf_ * pencil_blocks(a.p.seg, a.p.nseg, 1, nullptr),
+                    [&](int tw) { return nf_ * pencil_blocks(a.p.seg, a.p.nseg, tw, nullptr); });
     a.op = op;
     a.g = g_.kg;
     a.nmain = g_.nmain;
@@ -2251,7 +2312,7 @@ void Engine<T>::sync_from_spectra(bool mid) {
     }
     a.rows = g_.rows;
     a.nx = g_.nx;
-    a.TW = spread_tw(choose_tw(g_.nx, 1, sizeof(cpx<T>), 1), g_.rows);
+    a.TW = rows_tw(g_.rows);
     HIPCHK(launch_rows_sync<T>(a, st_));
     if (!mid || g_.ndim == 3) pencils(out, {}, 1, -1);
     if (!mid && g_.ndim == 3) pencils(out, {}, 2, -1);
@@ -2414,7 +2475,7 @@ void Engine<T>::etd_mid(const double* x, const double* v, int npt, const double*
         r.nmain = g_.nmain;
         r.rows = g_.rows;
         r.nx = g_.nx;
-        r.TW = spread_tw(choose_tw(g_.nx, 1, sizeof(cpx<T>), 1, 1), g_.rows);
+        r.TW = rows_tw(g_.rows, 1);
         HIPCHK(launch_rows_poly(r, st_));
         if (g_.ndim == 3) pencils(lines, {}, 1, -1);
         MidArgs<T> a = mid_args(kMidResidual);
@@ -3179,7 +3240,7 @@ void Engine<T>::adjoint(long nsteps, long every, const double* target, double* l
                 r.dnyq[0] = Lk.get() + g_.nmain;
                 r.rows = g_.rows;
                 r.nx = g_.nx;
-                r.TW = spread_tw(choose_tw(g_.nx, 1, sizeof(cpx<T>), 1), g_.rows);
+                r.TW = rows_tw(g_.rows);
                 HIPCHK(launch_rows_sync<T>(r, st_));
                 pencils({Lk.get()}, {}, 1, -1);
                 if (g_.ndim == 3) pencils({Lk.get()}, {}, 2, -1);
@@ -3368,7 +3429,7 @@ private:
                 b.p.arr[0][0] = d_.get();
                 b.p.seg[0] = s;
                 b.p.nseg = 1;
-                b.p.TW = choose_tw(bt.m, 1, sizeof(cpx<T>), s.sb == 1 ? 8 : 1);
+                b.p.TW = choose_tw(bt.m, sizeof(cpx<T>), s.sb == 1 ? 8 : 1);
                 b.m = bt.m;
                 b.chirp = bt.chirp.get();
                 b.filt = bt.filt.get();
@@ -3384,7 +3445,7 @@ private:
         a.arr[0][0] = d_.get();
         a.seg[0] = s;
         a.nseg = 1;
-        a.TW = choose_tw(n, 1, sizeof(cpx<T>), s.sb == 1 ? 8 : 1);
+        a.TW = choose_tw(n, sizeof(cpx<T>), s.sb == 1 ? 8 : 1);
         HIPCHK(launch_pencils<T>(a, n, dir, st_));
     }
     int ndim_;

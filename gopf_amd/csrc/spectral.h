@@ -130,8 +130,8 @@ struct PencilUpdateArgs {
     // rows of kMaxKTerms: indexed by power when dense, else by term (powers from denom / lin)
     const double* denom_sim = nullptr;
     const double* lin_sim = nullptr;
-    // tabulated multipliers (the persistent step): s1 = m1 - 1 and s2 = m2 / N of every
-    // k-point, in the layout of the state spectrum (main, nyq), and m1(0), m2(0) in FP64
+    // tabulated multipliers (or null: the pass computes them): s1 = m1 - 1 and s2 = m2 / N of
+    // every k-point, in the layout of the state spectrum (main, nyq), and m1(0), m2(0) in FP64
     cpx<T>* mtab[2] = {};
     double* m0 = nullptr;
 };
@@ -286,8 +286,10 @@ struct PersistLaunch {
                                            // on more than one XCD, the steps not run
 };
 bool persist_side(int n);  // the square sides with a persistent step
-// fills u.mtab and u.m0 with the update pass's multipliers (u.p set as for the pass, n = u.p.n)
-template <typename T> hipError_t launch_update_mult_table(const PencilUpdateArgs<T>& u, hipStream_t s);
+// tab and m0 = the update pass's multipliers (see PencilUpdateArgs::mtab) for the pass along
+// `axis` (1 = y, 2 = z), whose arithmetic they follow
+template <typename T> hipError_t launch_update_mult_table(const PencilUpdateArgs<T>& u, int axis, long nmain, long nk,
+                                                          cpx<T>* tab, double* m0, hipStream_t s);
 template <typename T> void persist_geometry(PersistLaunch<T>& L, int tw);  // threads and smem of L.n, L.mon
 template <typename T> hipError_t launch_fused_persist(const PersistLaunch<T>& L, hipStream_t s);
 

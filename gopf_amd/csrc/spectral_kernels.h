@@ -429,12 +429,10 @@ __device__ __forceinline__ void update_multipliers(const PencilUpdateArgs<T>& u,
 // UA is PencilUpdateArgs<T> for the plain kernel (its argument by value: read through a
 // reference, the kernel argument costs about ten more VGPRs, one wave per SIMD at 256) and
 // const PencilUpdateArgs<T>& for the grouped kernel (arguments read in place from global
-// memory: a copy would live in scratch).  EARLY: the line's loads are issued before the
-// multipliers are computed (their latency hidden behind that arithmetic, for two more lines
-// of registers), for launches whose passes are latency-bound.  MT: 0 the multipliers are
-// computed; 1 they are read from u.mtab / u.m0 with the line's loads; 2 they are computed,
-// written to u.mtab / u.m0, and the pass ends there (the table's own launch)
-template <typename T, int N, bool MON, typename UA = PencilUpdateArgs<T>, bool EARLY = false, int MT = 0>
+// memory: a copy would live in scratch).  MT: the multipliers are read from u.mtab / u.m0
+// instead of computed.  EARLY: the state's line (and the table's) is loaded with the source's,
+// before the transform, for two to four more lines of registers; otherwise after it, in chunks
+template <typename T, int N, bool MON, typename UA = PencilUpdateArgs<T>, bool EARLY = false, bool MT = false>
 __device__ __forceinline__ void pencil_update_body(UA u, int blk, int nblk, unsigned char* smem) {
     cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem);
     constexpr int V = 1;  // low-register schedule: two lines and the multipliers stay in registers
@@ -476,21 +474,24 @@ __device__ __forceinline__ void pencil_update_body(UA u, int blk, int nblk, unsi
     T s1a[E], s2a[E];
     double m1_0 = 1.0, m2_0 = 0.0;
     cpx<T> gs[E], c[E];
+    const cpx<T>* mtab = MT ? pick(u.mtab[0], u.mtab[1], ti.s) : nullptr;
     if constexpr (EARLY) {
         if (u.has_src) load_line<T, E>(gs, warr, base, ti.es, lm.t, TT, valid);
         load_line<T, E>(c, sarr, base, ti.es, lm.t, TT, valid);
     }
-    if constexpr (MT == 1) {
-        cpx<T> mt[E];
-        load_line<T, E>(mt, pick(u.mtab[0], u.mtab[1], ti.s), base, ti.es, lm.t, TT, valid);
+    if constexpr (MT) {
+        if constexpr (EARLY) {
+            cpx<T> mt[E];
+            load_line<T, E>(mt, mtab, base, ti.es, lm.t, TT, valid);
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                s1a[e] = mt[e].x;
+                s2a[e] = mt[e].y;
+            }
+        }
         if (has_k0) {
             m1_0 = u.m0[0];
             m2_0 = u.m0[1];
-        }
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            s1a[e] = mt[e].x;
-            s2a[e] = mt[e].y;
         }
     } else {
         const MultLine ml{lm.t, TT, nv, invv, fixed2};
@@ -500,40 +501,57 @@ __device__ __forceinline__ void pencil_update_body(UA u, int blk, int nblk, unsi
         else if (u.dense == 4) update_multipliers<T, E, 4>(u, ml, dsim, lsim, s1a, s2a, m1_0, m2_0);
         else update_multipliers<T, E, 0>(u, ml, dsim, lsim, s1a, s2a, m1_0, m2_0);
     }
-    if constexpr (MT == 2) {
-        cpx<T> mt[E];
-#pragma unroll
-        for (int e = 0; e < E; ++e) mt[e] = mk<T>(s1a[e], s2a[e]);
-        store_line<T, E>(mt, pick(u.mtab[0], u.mtab[1], ti.s), base, ti.es, lm.t, TT, valid);
-        if (has_k0) {
-            u.m0[0] = m1_0;
-            u.m0[1] = m2_0;
-        }
-        return;
-    }
-    // 2) explicit source: forward transform along this axis, scale by its multiplier
+    // 2) explicit source: forward transform along this axis, scaled by its multiplier
     double g0 = 0.0;
     if (u.has_src) {
         if constexpr (!EARLY) load_line<T, E>(gs, warr, base, ti.es, lm.t, TT, valid);
         line_fft<T, N, -1, V>(gs, lds + lm.off, lm.es, n, lm.t, a.tw);
         g0 = (double)gs[0].x;
+        if constexpr (!MT || EARLY) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) gs[e] = mk<T>(s2a[e] * gs[e].x, s2a[e] * gs[e].y);
+            for (int e = 0; e < E; ++e) gs[e] = mk<T>(s2a[e] * gs[e].x, s2a[e] * gs[e].y);
+        }
     } else {
 #pragma unroll
         for (int e = 0; e < E; ++e) gs[e] = mk<T>(T(0), T(0));
     }
     // 3) semi-implicit update of the state spectrum, which never leaves k-space
-    if constexpr (!EARLY) load_line<T, E>(c, sarr, base, ti.es, lm.t, TT, valid);
     double eg = 0.0;
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const cpx<T> cv = c[e];
+    // (g: the scaled source)
+    auto update = [&](int e, cpx<T> cv, T s1, cpx<T> g) {
         if (MON && valid) {
             const double fv = wrapk(lm.t + TT * e, nv) * invv;
             eg += wk * 4.0 * kPi * kPi * (fixed2 + fv * fv) * ((double)cv.x * (double)cv.x + (double)cv.y * (double)cv.y);
         }
-        c[e] = mk<T>(cv.x + (s1a[e] * cv.x + gs[e].x), cv.y + (s1a[e] * cv.y + gs[e].y));
+        c[e] = mk<T>(cv.x + (s1 * cv.x + g.x), cv.y + (s1 * cv.y + g.y));
+    };
+    if constexpr (MT && !EARLY) {
+        constexpr int C = (E % 5 == 0) ? 5 : (E % 4 == 0) ? 4 : (E % 7 == 0) ? 7 : 1;
+        cpx<T> sv[2][C], mt[2][C];
+        auto fetch = [&](int h, int e0) {
+#pragma unroll
+            for (int q = 0; q < C; ++q) {
+                const long off = base + (long)(lm.t + TT * (e0 + q)) * ti.es;
+                sv[h][q] = valid ? sarr[off] : mk<T>(T(0), T(0));
+                mt[h][q] = valid ? mtab[off] : mk<T>(T(0), T(0));
+            }
+        };
+        fetch(0, 0);
+#pragma unroll
+        for (int j = 0; j < E / C; ++j) {
+            if (j + 1 < E / C) fetch((j + 1) & 1, (j + 1) * C);
+            asm volatile("" ::: "memory");  // at most two chunks are live
+#pragma unroll
+            for (int q = 0; q < C; ++q) {
+                const int e = j * C + q;
+                const cpx<T> m = mt[j & 1][q];
+                update(e, sv[j & 1][q], m.x, mk<T>(m.y * gs[e].x, m.y * gs[e].y));
+            }
+        }
+    } else {
+        if constexpr (!EARLY) load_line<T, E>(c, sarr, base, ti.es, lm.t, TT, valid);
+#pragma unroll
+        for (int e = 0; e < E; ++e) update(e, c[e], s1a[e], gs[e]);
     }
     if (has_k0) {
         // k = 0 advances in FP64: the arrays hold c - mean, so their k = 0 coefficient stays 0
@@ -549,15 +567,24 @@ __device__ __forceinline__ void pencil_update_body(UA u, int blk, int nblk, unsi
         const double tot = block_sum(eg, red);
         if (threadIdx.x == 0) u.egrad_partial[blk] = tot / (u.scale * u.scale);
     }
-    // 4) the next step's row-pass input: the new state inverse-transformed along this axis
-    line_fft<T, N, +1, V>(c, lds + lm.off, lm.es, n, lm.t, a.tw);
+    // 4) the next step's row-pass input: the new state inverse-transformed along this axis.  With
+    // the chunked loads the twiddles and LDS addresses are formed anew rather than kept live from
+    // the forward transform (400 FP64 spilled); where the chain is the cost they are kept (128^2
+    // persistent step 12.4 against 13.8 us)
+    const cpx<T>* tw2 = a.tw;
+    int t2 = lm.t;
+    if constexpr (MT && !EARLY) asm volatile("" : "+s"(tw2), "+v"(t2));
+    line_fft<T, N, +1, V>(c, lds + lm.off, lm.es, n, t2, tw2);
     store_line<T, E>(c, warr, base, ti.es, lm.t, TT, valid);
 }
 
-template <typename T, int N, bool MON>
+// TAB: tabulated multipliers, everything loaded before the transform while a line's share of a
+// thread is at most 8 elements (the powers of two)
+template <typename T, int N, bool MON, bool TAB>
 __global__ void __launch_bounds__(kMaxBlock) k_pencil_update(PencilUpdateArgs<T> u) {
     extern __shared__ __align__(16) unsigned char smem[];
-    pencil_update_body<T, N, MON>(u, blockIdx.x, gridDim.x, smem);
+    constexpr bool kEarly = TAB && LineShape<N, 1>::E <= 8;
+    pencil_update_body<T, N, MON, PencilUpdateArgs<T>, kEarly, TAB>(u, blockIdx.x, gridDim.x, smem);
 }
 
 // x-rows: t fastest; the half spectrum split needs Z(k) and Z(n-k) from other threads
@@ -1471,8 +1498,13 @@ hipError_t launch_pencil_update_set(const PencilUpdateArgs<T>& u0, int n, hipStr
     if (u.egrad_partial) smem += (size_t)thr * sizeof(double);
     return dispatch_size<SET>(n, [&](auto NC) -> hipError_t {
         constexpr int NN = decltype(NC)::value;
-        if (u.egrad_partial) return launch_k(k_pencil_update<T, NN, true>, dim3(blocks), dim3(thr), smem, s, u);
-        return launch_k(k_pencil_update<T, NN, false>, dim3(blocks), dim3(thr), smem, s, u);
+        const dim3 g(blocks), b(thr);
+        if (u.mtab[0]) {
+            if (u.egrad_partial) return launch_k(k_pencil_update<T, NN, true, true>, g, b, smem, s, u);
+            return launch_k(k_pencil_update<T, NN, false, true>, g, b, smem, s, u);
+        }
+        if (u.egrad_partial) return launch_k(k_pencil_update<T, NN, true, false>, g, b, smem, s, u);
+        return launch_k(k_pencil_update<T, NN, false, false>, g, b, smem, s, u);
     });
 }
 

@@ -17,6 +17,7 @@
 // refuses a grid the device cannot hold at once.
 #pragma once
 
+#include "kspace.h"
 #include "spectral_kernels.h"
 
 namespace gpf {
@@ -117,39 +118,48 @@ __global__ void __launch_bounds__(kMaxBlock)
         }
         const PencilUpdateArgs<T>& u = P.u[s & 1];
         for (int b = pb; b < P.nblk_upd; b += (int)np) {
-            pencil_update_body<T, N, MON, const PencilUpdateArgs<T>&, true, 1>(u, b, P.nblk_upd, smem);
+            pencil_update_body<T, N, MON, const PencilUpdateArgs<T>&, true, true>(u, b, P.nblk_upd, smem);
             __syncthreads();
         }
         if (s + 1 < steps && !persist_barrier<LOCAL>(bar, gen, np, spin_limit, host_fail)) return;
     }
 }
 
-// the update pass's multipliers of every k-point (the pass in its table-writing form)
-template <typename T, int N>
-__global__ void __launch_bounds__(kMaxBlock) k_update_mult_table(PencilUpdateArgs<T> u) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    pencil_update_body<T, N, false, PencilUpdateArgs<T>, false, 2>(u, blockIdx.x, gridDim.x, smem);
+// the update pass's multipliers of every k-point, by the pass's own function
+template <typename T>
+__global__ void __launch_bounds__(256) k_update_mult_table(PencilUpdateArgs<T> u, int axis, long nmain, long nk,
+                                                           cpx<T>* __restrict__ tab, double* __restrict__ m0) {
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < nk; i += (long)gridDim.x * blockDim.x) {
+        int kx, ky, kz;
+        kcoords(u.g, i, nmain, kx, ky, kz);
+        const double fx = wrapk(kx, u.g.nx) * (1.0 / (double)u.g.nx), fy = wrapk(ky, u.g.ny) * (1.0 / (double)u.g.ny);
+        const double fz = (u.g.ndim == 3) ? wrapk(kz, u.g.nz) * (1.0 / (double)u.g.nz) : 0.0;
+        MultLine ml;
+        ml.t = (axis == 2) ? kz : ky;
+        ml.TT = 0;
+        ml.nv = (axis == 2) ? u.g.nz : u.g.ny;
+        ml.invv = 1.0 / (double)ml.nv;
+        ml.fixed2 = fx * fx + (axis == 1 ? 0.0 : fy * fy) + (axis == 2 ? 0.0 : fz * fz);
+        T s1, s2;
+        double m1 = 1.0, m2 = 0.0;
+        if (u.dense == 2) update_multipliers<T, 1, 2>(u, ml, nullptr, nullptr, &s1, &s2, m1, m2);
+        else if (u.dense == 4) update_multipliers<T, 1, 4>(u, ml, nullptr, nullptr, &s1, &s2, m1, m2);
+        else update_multipliers<T, 1, 0>(u, ml, nullptr, nullptr, &s1, &s2, m1, m2);
+        tab[i] = mk<T>(s1, s2);
+        if (i == 0) {
+            m0[0] = m1;
+            m0[1] = m2;
+        }
+    }
 }
 
 template <typename T>
-hipError_t launch_update_mult_table(const PencilUpdateArgs<T>& u0, hipStream_t s) {
-    PencilUpdateArgs<T> u = u0;
-    u.p.lpt = 1;
-    const long blocks = pencil_blocks(u.p.seg, u.p.nseg, u.p.TW, &u.p.tiles0);
-    const int thr = u.p.TW * threads_per_line(u.p.n, 1);
-    auto go = [&](auto NC) -> hipError_t {
-        constexpr int NN = decltype(NC)::value;
-        auto kern = k_update_mult_table<T, NN>;
-        hipLaunchKernelGGL(kern, dim3(blocks), dim3(thr), 0, s, u);
-        return hipGetLastError();
-    };
-    switch (u.p.n) {
-        case 32: return go(std::integral_constant<int, 32>{});
-        case 64: return go(std::integral_constant<int, 64>{});
-        case 128: return go(std::integral_constant<int, 128>{});
-        case 256: return go(std::integral_constant<int, 256>{});
-        default: return hipErrorInvalidValue;
-    }
+hipError_t launch_update_mult_table(const PencilUpdateArgs<T>& u, int axis, long nmain, long nk, cpx<T>* tab, double* m0,
+                                    hipStream_t s) {
+    const long blocks = (nk + 255) / 256;
+    hipLaunchKernelGGL(k_update_mult_table<T>, dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(256), 0, s, u, axis,
+                       nmain, nk, tab, m0);
+    return hipGetLastError();
 }
 
 // threads per block (tw lines of the schedule-1 transform) and dynamic LDS: the larger of the

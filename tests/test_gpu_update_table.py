@@ -1,0 +1,62 @@
+"""The fused step with tabulated update multipliers against the oracle, where the table, its chunked
+loads and the untuned launch layout can go wrong: lines of every count of elements per thread,
+tiles with one line or with lines past the end, an axis of two points, a filter set after the first
+steps (the table is rebuilt), the energy monitor, a mean that moves (k = 0 from the table).
+FP64 to 1e-10 max relative, FP32 to 1e-5 relative L2.
+"""
+import numpy as np
+import pytest
+
+import gopf_amd as G
+from gopf_amd import workloads as W
+from oracle import engine as E
+from oracle import parser as P
+
+pytestmark = pytest.mark.gpu
+
+AC = "dconc/dt = m2*conc - m4*conc^3 + mk*LAP conc"     # not conserved: the mean moves
+
+
+def models(dims, eq, seed):
+    n = int(np.prod(dims))
+    c0 = 0.5 + 0.1 * (np.random.default_rng(seed).random(n) - 0.5)
+    pm, om = G.Model(), P.Model()
+    pm.AddField("conc", c0)
+    om.add_field("conc", n)
+    for k, v in W.ch_scalars(1.0, 1.0).items():
+        pm.AddScalar(k, v)
+        om.add_scalar(k, v)
+    pm.AddEquation(eq)
+    om.add_equation(eq)
+    pm.Init()
+    om.init()
+    return pm, om, c0
+
+
+def close(got, ref, precision):
+    if precision == "fp64":
+        return np.abs(got - ref).max() <= 1e-10 * np.abs(ref).max()
+    return np.linalg.norm(got - ref) <= 1e-5 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("eq", [W.CH_EQUATION, AC], ids=["ch", "ac"])
+@pytest.mark.parametrize("dims", [[2, 16], [100, 12], [112, 20], [400, 10], [250, 64], [512, 30], [33, 50], [768, 8],
+                                  [20, 20, 20], [24, 24, 24], [9, 9, 9]])
+def test_fused_step_with_table(dims, eq, precision):
+    pm, om, c0 = models(dims, eq, 3)
+    s = G.Solver(pm, dims, 0.05, precision=precision)
+    assert s.fused
+    o = E.OracleSolver(om, dims, {"conc": c0}, 0.05)
+    s.MonitorEnergy(W.CH_BULK_POLY, 1.0)
+    s.Propagate(13)
+    o.stepper_propagate(13)
+    assert close(s.Field(0).real, o.field("conc").real, precision)
+    energy, mass = s.EnergySeries()
+    assert energy.size == 13 and abs(mass[0] - c0.sum()) <= 1e-6 * abs(c0.sum())
+    # a filter from here on
+    s.SetFilter(G.NewVandeven(4))
+    f = E.OracleSolver(om, dims, {"conc": o.field("conc").real}, 0.05, filter_order=4)
+    s.Propagate(5)
+    f.stepper_propagate(5)
+    assert close(s.Field(0).real, f.field("conc").real, precision)
