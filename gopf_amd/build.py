@@ -25,7 +25,8 @@ SOURCES = ["spectral_ext_mid.hip", "spectral_ext_mid64.hip", "spectral_mid.hip",
            "spectral_pencils_fwd64.hip", "spectral_pencils_inv64.hip", "spectral_sync64.hip", "spectral_r2c64.hip",
            "spectral_c2r64.hip", "spectral_update64.hip", "spectral_rows64.hip", "spectral_group.hip",
            "spectral_group64.hip", "spectral_persist.hip", "spectral_persist64.hip", "spectral_pencils.hip",
-           "spectral_pencils64.hip", "spectral_rowpoly.hip", "spectral.hip", "engine.hip",
+           "spectral_pencils64.hip", "spectral_rowpoly.hip", "spectral_adjoint.hip", "spectral_adjoint64.hip",
+           "spectral.hip", "engine.hip",
            "pointwise.hip", "batch.hip", "krylov.hip", "io.hip", "reduce.hip", "model.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"

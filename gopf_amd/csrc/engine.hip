@@ -45,6 +45,7 @@
 #include "model.h"
 #include "pointwise.h"
 #include "spectral.h"
+#include "spectral_adjoint.h"
 #include "spectral_mid.h"
 #include "spectral_rowpoly.h"
 
@@ -595,6 +596,16 @@ private:
     int rows_var_ = 0;  // transform schedule of the row pass (0 plain, 1 low-register)
     int lpt_pf_ = 1, lpt_pi_ = 1;  // lines per thread of the forward / inverse pencil passes
     T* c_out_ = nullptr;           // when set, the next row pass also writes the real field c here
+    // when set, the next step reads its state and mean from these and writes the new ones to the
+    // others (the adjoint's stored states)
+    const cpx<T>* s_in_ = nullptr;
+    cpx<T>* s_out_ = nullptr;
+    double *mean_in_ = nullptr, *mean_out_ = nullptr;
+    // the adjoint's checkpoints and segment storage: one allocation each, kept between calls up to
+    // kAdjKeep bytes
+    static constexpr size_t kAdjKeep = (size_t)1 << 30;
+    Buf<cpx<T>> adj_k_;
+    Buf<T> adj_r_;
     int var_pf_ = 0, var_pi_ = 0;  // transform schedules of the forward / inverse pencil passes
     // 3D: axis of the fused forward-update-inverse pass (2 = z, 1 = y); the other
     // of y / z is transformed forward before and inverse after it
@@ -1621,9 +1632,15 @@ void Engine<T>::prepare_fused(long upcoming) {
 // 64 threads); the last step of the sequence writes its own slot with a launch of its own.
 template <typename T>
 void Engine<T>::enqueue_fused(int pos, int count) {
-    RowFusedArgs<T> ra = rows_args(W_.get(), mean_.get(), tw_rows_, rows_var_);
+    double* mean = mean_in_ ? mean_in_ : mean_.get();
+    RowFusedArgs<T> ra = rows_args(W_.get(), mean, tw_rows_, rows_var_);
     const int nu = axis_len(upd_axis());
-    PencilUpdateArgs<T> u = update_args(S_.get(), W_.get(), mean_.get(), tw_pu_);
+    PencilUpdateArgs<T> u = update_args(s_out_ ? s_out_ : S_.get(), W_.get(), mean, tw_pu_);
+    if (s_in_) {
+        u.p.src[0][0] = s_in_;
+        u.p.src[0][1] = s_in_ + g_.nmain;
+        u.mean_out = mean_out_;
+    }
     const double ceg = 0.5 * mon_kappa_ / (double)g_.n;
     const long cur = pos & 1, prev = (pos + 1) & 1;
     const bool rows_pass = fp_.has_src || mon_;
@@ -3070,9 +3087,22 @@ void Engine<T>::adjoint(long nsteps, long every, const double* target, double* l
     if (nscal < 0 || nscal > kMaxAdjScalars) throw Error(GPF_EINVAL, "at most 8 scalars per adjoint run");
     if (nscal > 0 && (!names || !grad_scalars)) throw Error(GPF_EINVAL, "scalar names and output are required");
     if (autotune_ && !tuned_) autotune();
-    const bool mon = mon_, timing = timing_;
+    // the segments are captured as graphs: no monitor, no per-pass events; the settings and the
+    // step's normal state come back however the run ends
+    struct Settings {
+        Engine* e;
+        bool mon, timing;
+        ~Settings() {
+            e->mon_ = mon;
+            e->timing_ = timing;
+            e->c_out_ = nullptr;
+            e->s_in_ = nullptr;
+            e->s_out_ = nullptr;
+            e->mean_in_ = e->mean_out_ = nullptr;
+        }
+    } settings{this, mon_, timing_};
     mon_ = false;
-    timing_ = false;  // the segments are captured as graphs: no per-pass events
+    timing_ = false;
     const long n = g_.n, nk = g_.nk;
     // parameter tables: derivative of D, E (per LAP power) and of g (per power of c)
     std::vector<double> dcoef((size_t)std::max(nscal, 1) * 2 * kMaxKTerms, 0.0);
@@ -3115,19 +3145,25 @@ void Engine<T>::adjoint(long nsteps, long every, const double* target, double* l
         HIPCHK(hipStreamSynchronize(st_));
     }
     // forward sweep with checkpoints of the fused state
+    // checkpoints, the segment's state spectra S_n and real fields c_n in two allocations (with one
+    // per array, 200 hipMalloc and hipFree calls were 58 of the 88 ms of a 400-step run at 512^2);
+    // strides of 32 elements keep every array's 16-byte alignment
     const long nck = (nsteps + every - 1) / every;
-    std::vector<Buf<cpx<T>>> ck;
+    const long seglen = std::min(every, nsteps);
+    const bool need_real = fp_.has_src;
+    const long ks = (nk + 31) / 32 * 32, rstr = (n + 31) / 32 * 32;
+    const size_t want_k = (size_t)(nck + seglen + 1) * ks, want_r = need_real ? (size_t)seglen * rstr : 1;
+    if (adj_k_.size() < want_k) adj_k_.alloc(want_k);
+    if (adj_r_.size() < want_r) adj_r_.alloc(want_r);
+    auto ck = [&](long i) { return adj_k_.get() + i * ks; };
+    auto SS = [&](long i) { return adj_k_.get() + (nck + i) * ks; };
+    auto R = [&](long i) { return adj_r_.get() + i * rstr; };
     Buf<double> ckmean(nck);
     for (long s = 0; s < nsteps; s += every) {
-        ck.emplace_back(nk);
-        HIPCHK(hipMemcpyAsync(ck.back().get(), S_.get(), nk * sizeof(cpx<T>), hipMemcpyDeviceToDevice, st_));
+        HIPCHK(hipMemcpyAsync(ck(s / every), S_.get(), nk * sizeof(cpx<T>), hipMemcpyDeviceToDevice, st_));
         HIPCHK(hipMemcpyAsync(ckmean.get() + s / every, mean_.get(), sizeof(double), hipMemcpyDeviceToDevice, st_));
         steps(std::min(every, nsteps - s));
     }
-    Buf<cpx<T>> Sf(nk);
-    Buf<double> meanf(1);
-    HIPCHK(hipMemcpyAsync(Sf.get(), S_.get(), nk * sizeof(cpx<T>), hipMemcpyDeviceToDevice, st_));
-    HIPCHK(hipMemcpyAsync(meanf.get(), mean_.get(), sizeof(double), hipMemcpyDeviceToDevice, st_));
     // loss and lam_T = 2 (c_T - target), in FP64 on the host
     std::vector<double> cT(2 * n);
     get_field(0, cT.data());
@@ -3144,20 +3180,23 @@ void Engine<T>::adjoint(long nsteps, long every, const double* target, double* l
     *loss = js + jc;
     Buf<T> lam(n), pr(n), qr(n);
     HIPCHK(hipMemcpyAsync(lam.get(), lamT.data(), n * sizeof(T), hipMemcpyHostToDevice, st_));
-    // segment storage: the state spectra S_n (and means) and the real fields c_n that the
-    // recomputed row passes write as a by-product
-    const long seglen = std::min(every, nsteps);
-    const bool need_real = fp_.has_src;
-    std::vector<Buf<cpx<T>>> SS;
-    std::vector<Buf<T>> R;
-    for (long i = 0; i <= seglen; ++i) SS.emplace_back(nk);
-    if (need_real)
-        for (long i = 0; i < seglen; ++i) R.emplace_back(n);
     Buf<double> segmean(seglen + 1);
     bool any_g = false;
     for (int q = 0; q < nscal; ++q) any_g |= !dpoly[q].empty();
-    Buf<cpx<T>> Lk(nk), Pk(nk), Qk(nk);
-    const long nblk = std::max(1L, std::min((nk + 255) / 256, 1024L));
+    Buf<cpx<T>> Lk(nk);
+    cpx<T>* Pk = kscratch(0);
+    cpx<T>* Qk = kscratch(1);
+    AdjMidArgs<T> am;
+    {
+        const int axis = mid_axis(), nl = axis_len(axis);
+        am.p.tw = tw(nl);
+        am.p.seg[0] = (axis == 2) ? seg_z_main(g_) : seg_y_main(g_);
+        am.p.seg[1] = (axis == 2) ? seg_z_nyq(g_) : seg_y_nyq(g_);
+        am.p.nseg = 2;
+        am.p.TW = fit_tw(nl, sizeof(cpx<T>), 1, true, pencil_blocks(am.p.seg, am.p.nseg, 1, nullptr),
+                         [&](int t) { return pencil_blocks(am.p.seg, am.p.nseg, t, nullptr); });
+    }
+    const long nblk = adj_mid_blocks<T>(am);
     const long nblk_r = std::max(1L, std::min((n + 255) / 256, 1024L));
     // per-block partial sums, accumulated in place across the reverse sweep (each block owns
     // its slot; launches are ordered on the stream) and reduced once at the end
@@ -3166,7 +3205,7 @@ void Engine<T>::adjoint(long nsteps, long every, const double* target, double* l
     HIPCHK(hipMemsetAsync(acc.get(), 0, std::max(nscal, 1) * sizeof(double), st_));
     HIPCHK(hipMemsetAsync(partial_k.get(), 0, std::max(nscal, 1) * nblk * sizeof(double), st_));
     HIPCHK(hipMemsetAsync(partial_r.get(), 0, std::max(nscal, 1) * nblk_r * sizeof(double), st_));
-    AdjArgs<T> a;
+    AdjArgs<T>& a = am.a;
     a.g = g_.kg;
     a.nmain = g_.nmain;
     a.nk = nk;
@@ -3176,30 +3215,42 @@ void Engine<T>::adjoint(long nsteps, long every, const double* target, double* l
     a.src_lap = fp_.src_lap;
     a.filter = has_filter_ ? filter_.get() : nullptr;
     a.lam = Lk.get();
-    a.P = Pk.get();
-    a.Q = Qk.get();
+    a.P = Pk;
+    a.Q = Qk;
     a.nscal = nscal;
     a.dcoef = d_dcoef.get();
     a.cscale = (double)n;
     a.partial = partial_k.get();
     a.inv_n = 1.0 / (double)n;
+    const bool grad = nscal > 0 && (need_c1 || need_c0);
+    Buf<double2> mtab(nk), gtab(grad ? (size_t)nscal * nk : 1);
+    {
+        AdjArgs<T> ta = a;
+        if (!grad) ta.nscal = 0;
+        HIPCHK(launch_adj_tables<T>(ta, mtab.get(), gtab.get(), st_));
+    }
+    am.t.m = mtab.get();
+    am.t.g = gtab.get();
     const int ndg = (int)dg.size();
     // one segment's recompute and reverse sweep; device pointers depend only on the step's
-    // offset in its segment, so a full segment can be captured once and replayed (copies
-    // are kernels, nothing is allocated)
-    auto copy_k = [&](cpx<T>* dst, const cpx<T>* src) {
-        HIPCHK(launch_copy<T>(reinterpret_cast<const T*>(src), reinterpret_cast<T*>(dst), 2 * nk, st_));
-    };
+    // offset in its segment, so a full segment can be captured once and replayed (nothing is
+    // allocated).  Each recomputed step reads S_n and writes S_{n+1} (and the means) in place
+    // among the stored states, and its row pass writes c_n.
     auto recompute = [&](long len) {
         for (long k = 0; k < len; ++k) {
-            copy_k(SS[k].get(), S_.get());
-            if (split_mean_) HIPCHK(launch_copy<double>(mean_.get(), segmean.get() + k, 1, st_));
-            c_out_ = need_real ? R[k].get() : nullptr;
+            c_out_ = need_real ? R(k) : nullptr;
+            s_in_ = SS(k);
+            s_out_ = SS(k + 1);
+            if (split_mean_) {
+                mean_in_ = segmean.get() + k;
+                mean_out_ = segmean.get() + k + 1;
+            }
             fused_step();
-            c_out_ = nullptr;
         }
-        copy_k(SS[len].get(), S_.get());
-        if (split_mean_) HIPCHK(launch_copy<double>(mean_.get(), segmean.get() + len, 1, st_));
+        c_out_ = nullptr;
+        s_in_ = nullptr;
+        s_out_ = nullptr;
+        mean_in_ = mean_out_ = nullptr;
     };
     // Unless a scalar's gradient needs the source-derivative sums <q, dg/ds(c_n)> (kept in
     // k_adj_lambda), the inverse rows of P and Q, lam_n = p + g'(c_n) q and the forward
@@ -3208,27 +3259,23 @@ void Engine<T>::adjoint(long nsteps, long every, const double* target, double* l
     const bool fuse_rev = !(nscal > 0 && any_g) && ndg <= kMaxPoly;
     auto reverse = [&](long len) {
         for (long k = len - 1; k >= 0; --k) {
-            const T* cn = need_real ? R[k].get() : nullptr;
-            if (!fuse_rev) r2c({lam.get()}, {Lk.get()}, T(1));
-            if (nscal > 0 && (need_c1 || need_c0)) {
-                // P, Q and the derivatives of D and E against the transforms of c_{n+1} and c_n
-                a.C1 = need_c1 ? SS[k + 1].get() : nullptr;
-                a.C0 = need_c0 ? SS[k].get() : nullptr;
-                a.mean1 = split_mean_ ? segmean.get() + (k + 1) : nullptr;
-                a.mean0 = split_mean_ ? segmean.get() + k : nullptr;
-                HIPCHK(launch_adj_grad<T>(a, nblk, st_));
-            } else {
-                HIPCHK(launch_adj_mult<T>(a, st_));
-            }
+            const T* cn = need_real ? R(k) : nullptr;
+            // along the last axis: lam forward, P and Q with the derivatives of D and E against the
+            // transforms of c_{n+1} and c_n, P and Q back
+            if (!fuse_rev) r2c({lam.get()}, {Lk.get()}, T(1), nullptr, false);
+            a.C1 = grad && need_c1 ? SS(k + 1) : nullptr;
+            a.C0 = grad && need_c0 ? SS(k) : nullptr;
+            a.mean1 = split_mean_ ? segmean.get() + (k + 1) : nullptr;
+            a.mean0 = split_mean_ ? segmean.get() + k : nullptr;
+            HIPCHK(launch_adj_mid<T>(am, axis_len(mid_axis()), st_));
             if (fuse_rev) {
-                if (g_.ndim == 3) pencils({Pk.get(), Qk.get()}, {}, 2, +1);
-                pencils({Pk.get(), Qk.get()}, {}, 1, +1);
+                if (g_.ndim == 3) pencils({Pk, Qk}, {}, 1, +1);
                 RowSyncArgs<T> r;
                 r.tw = tw(g_.nx);
-                r.fmain[0] = Pk.get();
-                r.fnyq[0] = Pk.get() + g_.nmain;
-                r.fmain[1] = Qk.get();
-                r.fnyq[1] = Qk.get() + g_.nmain;
+                r.fmain[0] = Pk;
+                r.fnyq[0] = Pk + g_.nmain;
+                r.fmain[1] = Qk;
+                r.fnyq[1] = Qk + g_.nmain;
                 r.fout[0] = lam.get();
                 r.scale = T(1) / (T)n;
                 r.mode = 2;
@@ -3242,11 +3289,10 @@ void Engine<T>::adjoint(long nsteps, long every, const double* target, double* l
                 r.nx = g_.nx;
                 r.TW = rows_tw(g_.rows);
                 HIPCHK(launch_rows_sync<T>(r, st_));
-                pencils({Lk.get()}, {}, 1, -1);
-                if (g_.ndim == 3) pencils({Lk.get()}, {}, 2, -1);
+                if (g_.ndim == 3) pencils({Lk.get()}, {}, 1, -1);
                 continue;
             }
-            c2r({Pk.get(), Qk.get()}, {pr.get(), qr.get()}, T(1) / (T)n);
+            c2r({Pk, Qk}, {pr.get(), qr.get()}, T(1) / (T)n, nullptr, false);
             if (need_real) {
                 // lam_n = p + g'(c_n) q, and the source derivatives <q, dg/ds(c_n)> in real space
                 HIPCHK(launch_adj_lambda<T>(pr.get(), qr.get(), cn, ndg, d_dg.get(), lam.get(), n, any_g ? nscal : 0,
@@ -3267,14 +3313,14 @@ void Engine<T>::adjoint(long nsteps, long every, const double* target, double* l
         HIPCHK(e);
         return ge;
     };
-    if (fuse_rev) r2c({lam.get()}, {Lk.get()}, T(1));
+    if (fuse_rev) r2c({lam.get()}, {Lk.get()}, T(1), nullptr, false);
     hipGraphExec_t g_rec = nullptr, g_rev = nullptr;
     bool warm = false;  // the first segment runs eagerly: it creates every lazily built table
     for (long seg = nck - 1; seg >= 0; --seg) {
         const long s0 = seg * every, s1 = std::min(nsteps, s0 + every), len = s1 - s0;
-        HIPCHK(hipMemcpyAsync(S_.get(), ck[seg].get(), nk * sizeof(cpx<T>), hipMemcpyDeviceToDevice, st_));
-        HIPCHK(hipMemcpyAsync(mean_.get(), ckmean.get() + seg, sizeof(double), hipMemcpyDeviceToDevice, st_));
-        prime();
+        HIPCHK(hipMemcpyAsync(SS(0), ck(seg), nk * sizeof(cpx<T>), hipMemcpyDeviceToDevice, st_));
+        HIPCHK(hipMemcpyAsync(segmean.get(), ckmean.get() + seg, sizeof(double), hipMemcpyDeviceToDevice, st_));
+        pencils({W_.get()}, {SS(0)}, upd_axis(), +1);
         if (warm && len == every && len >= 2) {
             if (!g_rec) g_rec = capture([&] { recompute(len); });
             HIPCHK(hipGraphLaunch(g_rec, st_));
@@ -3298,15 +3344,15 @@ void Engine<T>::adjoint(long nsteps, long every, const double* target, double* l
     HIPCHK(hipMemcpyAsync(hl.data(), lam.get(), n * sizeof(T), hipMemcpyDeviceToHost, st_));
     std::vector<double> hs(std::max(nscal, 1));
     HIPCHK(hipMemcpyAsync(hs.data(), acc.get(), hs.size() * sizeof(double), hipMemcpyDeviceToHost, st_));
-    HIPCHK(hipMemcpyAsync(S_.get(), Sf.get(), nk * sizeof(cpx<T>), hipMemcpyDeviceToDevice, st_));
-    HIPCHK(hipMemcpyAsync(mean_.get(), meanf.get(), sizeof(double), hipMemcpyDeviceToDevice, st_));
-    prime();
+    prime();  // S_ and the mean are c_T's still; the work array held the recomputed steps'
     HIPCHK(hipStreamSynchronize(st_));
+    if (adj_k_.size() * sizeof(cpx<T>) + adj_r_.size() * sizeof(T) > kAdjKeep) {
+        adj_k_ = Buf<cpx<T>>();
+        adj_r_ = Buf<T>();
+    }
     if (grad_field)
         for (long i = 0; i < n; ++i) grad_field[i] = (double)hl[i];
     for (int s = 0; s < nscal; ++s) grad_scalars[s] = hs[s];
-    mon_ = mon;
-    timing_ = timing;
 }
 
 // ---------------------------------------------------------------------------

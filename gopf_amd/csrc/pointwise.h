@@ -244,11 +244,11 @@ struct AdjArgs {
     KPoly denom, lin;          // D(k), E(k)
     int src_lap = 0;
     const double* filter = nullptr;
-    // k_adj_mult: P = m1 Lam, Q = m2 Lam with m1 = A (1 + dt E), m2 = A dt L^src_lap, A = sigma / (1 - dt D)
+    // P = m1 Lam, Q = m2 Lam with m1 = A (1 + dt E), m2 = A dt L^src_lap, A = sigma / (1 - dt D)
     const cpx<T>* lam = nullptr;
     cpx<T>* P = nullptr;
     cpx<T>* Q = nullptr;
-    // k_adj_grad: P and Q as k_adj_mult, and per scalar s the block sums of
+    // and per scalar s the block sums of
     // w Re(conj(Lam) [dt dD_s C1 / (1 - dt D) + A dt dE_s C0]) / N added to partial[s][block], with
     // dD_s = sum_t dcoef[s][0][t] L^denom.pow[t], dE_s = sum_t dcoef[s][1][t] L^lin.pow[t] and the
     // transforms C1 = FFT(c_{n+1}), C0 = FFT(c_n) given as state spectra: C = cscale S, plus
@@ -264,8 +264,9 @@ struct AdjArgs {
     double inv_n = 1.0;
 };
 
-template <typename T> hipError_t launch_adj_mult(const AdjArgs<T>& a, hipStream_t s);
-template <typename T> hipError_t launch_adj_grad(const AdjArgs<T>& a, long nblocks, hipStream_t s);
+// m[k] = (m1, m2); g[s nk + k] = the weights (dt dD_s / (1 - dt D), A dt dE_s) of C1 and C0 in scalar s's
+// sum, times w / N
+template <typename T> hipError_t launch_adj_tables(const AdjArgs<T>& a, double2* m, double2* g, hipStream_t s);
 // out = p + h(c) q with h(c) = sum_k dpoly[k] c^k; a null p reads as 0 and a null q as 1
 // (the adjoint's lam_n = p + g'(c_n) q, and plain polynomial evaluation).  With nscal > 0
 // it also adds, per scalar s, the block sums of q(x) sum_k spoly[s][k] c(x)^k to

@@ -739,77 +739,31 @@ __global__ void __launch_bounds__(kRedThreads) k_reduce2(const double* a, long n
     if (threadIdx.x == 0) out[0] = ca * x + cb * y;
 }
 
-__device__ __forceinline__ void adj_coeffs(const KGrid& g, long i, long nmain, double dt, const KPoly& den,
-                                           const KPoly& lin, int src_lap, const double* filter, double& L, double& A,
-                                           double& Ainv, double& m1, double& m2, double& w) {
-    int kx, ky, kz;
-    kcoords(g, i, nmain, kx, ky, kz);
-    double f[3];
-    ref_freq(g, kx, ky, kz, f);
-    const double f2 = f[0] * f[0] + f[1] * f[1] + f[2] * f[2];
-    L = -(4.0 * kPi * kPi) * f2;
-    double D = 0.0, E = 0.0;
-    for (int t = 0; t < den.n; ++t) D += den.coef[t] * ipow(L, den.pow[t]);
-    for (int t = 0; t < lin.n; ++t) E += lin.coef[t] * ipow(L, lin.pow[t]);
-    Ainv = 1.0 / (1.0 - dt * D);
-    A = Ainv;
-    if (filter) A *= vandeven(filter, sqrt(f2) * 2.0 / kPi);
-    m1 = A * (1.0 + dt * E);
-    m2 = A * dt * ipow(L, src_lap);
-    w = (kx == 0 || 2 * kx == g.nx) ? 1.0 : 2.0;
-}
-
+// the reverse step's multipliers and, per scalar, the weights of its sums (AdjArgs), of every k-point
 template <typename T>
-__global__ void k_adj_mult(AdjArgs<T> a) {
+__global__ void __launch_bounds__(256) k_adj_tables(AdjArgs<T> a, double2* __restrict__ m, double2* __restrict__ g) {
     for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < a.nk; i += (long)gridDim.x * blockDim.x) {
-        double L, A, Ainv, m1, m2, w;
-        adj_coeffs(a.g, i, a.nmain, a.dt, a.denom, a.lin, a.src_lap, a.filter, L, A, Ainv, m1, m2, w);
-        const cpx<T> l = a.lam[i];
-        a.P[i] = mk<T>((T)(m1 * (double)l.x), (T)(m1 * (double)l.y));
-        a.Q[i] = mk<T>((T)(m2 * (double)l.x), (T)(m2 * (double)l.y));
-    }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_adj_grad(AdjArgs<T> a) {
-    __shared__ double red[256];
-    double acc[kMaxAdjScalars];
-    for (int s = 0; s < kMaxAdjScalars; ++s) acc[s] = 0.0;
-    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < a.nk; i += (long)gridDim.x * blockDim.x) {
-        double L, A, Ainv, m1, m2, w;
-        adj_coeffs(a.g, i, a.nmain, a.dt, a.denom, a.lin, a.src_lap, a.filter, L, A, Ainv, m1, m2, w);
-        const cpx<T> l = a.lam[i];
-        a.P[i] = mk<T>((T)(m1 * (double)l.x), (T)(m1 * (double)l.y));
-        a.Q[i] = mk<T>((T)(m2 * (double)l.x), (T)(m2 * (double)l.y));
-        double c1x = 0.0, c1y = 0.0, c0x = 0.0, c0y = 0.0;
-        if (a.C1) {
-            c1x = a.cscale * (double)a.C1[i].x;
-            c1y = a.cscale * (double)a.C1[i].y;
-            if (i == 0 && a.mean1) c1x += a.cscale * *a.mean1;
-        }
-        if (a.C0) {
-            c0x = a.cscale * (double)a.C0[i].x;
-            c0y = a.cscale * (double)a.C0[i].y;
-            if (i == 0 && a.mean0) c0x += a.cscale * *a.mean0;
-        }
-        // Re(conj(l) z) = l.x z.x + l.y z.y
-        const double lc1 = (double)l.x * c1x + (double)l.y * c1y;
-        const double lc0 = (double)l.x * c0x + (double)l.y * c0y;
-#pragma unroll
-        for (int s = 0; s < kMaxAdjScalars; ++s) {
-            if (s >= a.nscal) break;
+        int kx, ky, kz;
+        kcoords(a.g, i, a.nmain, kx, ky, kz);
+        double f[3];
+        ref_freq(a.g, kx, ky, kz, f);
+        const double f2 = f[0] * f[0] + f[1] * f[1] + f[2] * f[2];
+        const double L = -(4.0 * kPi * kPi) * f2;
+        double D = 0.0, E = 0.0;
+        for (int t = 0; t < a.denom.n; ++t) D += a.denom.coef[t] * ipow(L, a.denom.pow[t]);
+        for (int t = 0; t < a.lin.n; ++t) E += a.lin.coef[t] * ipow(L, a.lin.pow[t]);
+        const double Ainv = 1.0 / (1.0 - a.dt * D);
+        double A = Ainv;
+        if (a.filter) A *= vandeven(a.filter, sqrt(f2) * 2.0 / kPi);
+        m[i] = make_double2(A * (1.0 + a.dt * E), A * a.dt * ipow(L, a.src_lap));
+        const double w = ((kx == 0 || 2 * kx == a.g.nx) ? 1.0 : 2.0) * a.inv_n;
+        for (int s = 0; s < a.nscal; ++s) {
             const double* dc = a.dcoef + (long)s * 2 * kMaxKTerms;
             double dD = 0.0, dE = 0.0;
             for (int t = 0; t < a.denom.n; ++t) dD += dc[t] * ipow(L, a.denom.pow[t]);
             for (int t = 0; t < a.lin.n; ++t) dE += dc[kMaxKTerms + t] * ipow(L, a.lin.pow[t]);
-            acc[s] += w * (Ainv * a.dt * dD * lc1 + A * a.dt * dE * lc0);
+            g[(long)s * a.nk + i] = make_double2(w * Ainv * a.dt * dD, w * A * a.dt * dE);
         }
-    }
-#pragma unroll
-    for (int s = 0; s < kMaxAdjScalars; ++s) {
-        if (s >= a.nscal) break;  // uniform over the block
-        const double tot = block_sum(acc[s], red);
-        if (threadIdx.x == 0) a.partial[(long)s * gridDim.x + blockIdx.x] += tot * a.inv_n;
     }
 }
 
@@ -1218,13 +1172,8 @@ hipError_t launch_copy_bw(const float* src, float* dst, long n, hipStream_t s) {
 }
 
 template <typename T>
-hipError_t launch_adj_mult(const AdjArgs<T>& a, hipStream_t s) {
-    hipLaunchKernelGGL(k_adj_mult<T>, dim3(grid_for(a.nk)), dim3(256), 0, s, a);
-    return hipGetLastError();
-}
-template <typename T>
-hipError_t launch_adj_grad(const AdjArgs<T>& a, long nblocks, hipStream_t s) {
-    hipLaunchKernelGGL(k_adj_grad<T>, dim3((unsigned)nblocks), dim3(256), 0, s, a);
+hipError_t launch_adj_tables(const AdjArgs<T>& a, double2* m, double2* g, hipStream_t s) {
+    hipLaunchKernelGGL(k_adj_tables<T>, dim3(grid_for(a.nk)), dim3(256), 0, s, a, m, g);
     return hipGetLastError();
 }
 template <typename T>
@@ -1275,8 +1224,7 @@ hipError_t launch_reduce2(const double* a, long na, double ca, const double* b, 
     template hipError_t launch_real_sums<T>(const T*, long, double, int, const double*, double*, double*,     \
                                             long, hipStream_t);                                               \
     template hipError_t launch_kgrad_energy<T>(const cpx<T>*, KGrid, long, long, double*, long, hipStream_t); \
-    template hipError_t launch_adj_mult<T>(const AdjArgs<T>&, hipStream_t);                                  \
-    template hipError_t launch_adj_grad<T>(const AdjArgs<T>&, long, hipStream_t);                            \
+    template hipError_t launch_adj_tables<T>(const AdjArgs<T>&, double2*, double2*, hipStream_t);             \
     template hipError_t launch_adj_lambda<T>(const T*, const T*, const T*, int, const double*, T*, long, int, \
                                              const double*, double*, long, hipStream_t);
 GPF_INST(float)

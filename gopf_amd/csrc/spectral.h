@@ -120,6 +120,9 @@ struct PencilUpdateArgs {
     const double* filter = nullptr;      // Vandeven table (1000 entries) or null
     double* mean = nullptr;              // FP64 k = 0 mode: the field mean (in/out), or null when the
                                          // k = 0 coefficient is carried by the arrays themselves
+    // the state is read from p.src[0] and the mean from `mean` where these are set, and the new ones
+    // written to arr[0] and mean_out: a sequence of stored states needs no copies
+    double* mean_out = nullptr;
     double* egrad_partial = nullptr;     // per-block FP64 sum of w (2 pi |f|)^2 |FFT(c)|^2 or null
     // dense form (dense = 2 or 4: every LAP power of D, E and the source is at most that
     // degree): D(L) = sum_p dd[p] L^p, E(L) = sum_p dl[p] L^p; 0: the term lists above

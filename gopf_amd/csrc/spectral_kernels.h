@@ -444,7 +444,12 @@ __device__ __forceinline__ void pencil_update_body(UA u, int blk, int nblk, unsi
     const LineMap lm = line_map(ti.es == 1, a.TW, TT, n);
     const bool valid = lm.l < ti.nvalid;
     const long base = ti.base + (long)lm.l * ti.sb;
-    cpx<T>* sarr = pick(a.arr[0][0], a.arr[0][1], ti.s);
+    cpx<T>* sout = pick(a.arr[0][0], a.arr[0][1], ti.s);
+    // a separate input state (PencilUpdateArgs::mean_out) with the arguments by value only: the
+    // persistent step does not pay for the choice
+    constexpr bool kApart = !std::is_reference<UA>::value;
+    const cpx<T>* ssrc = kApart ? pick(a.src[0][0], a.src[0][1], ti.s) : nullptr;
+    const cpx<T>* sarr = ssrc ? ssrc : sout;
     cpx<T>* warr = pick(a.arr[1][0], a.arr[1][1], ti.s);
     const double inx = 1.0 / (double)u.g.nx, iny = 1.0 / (double)u.g.ny, inz = 1.0 / (double)u.g.nz;
     // 1) k-space multipliers of this thread's elements, computed before any data is
@@ -557,10 +562,10 @@ __device__ __forceinline__ void pencil_update_body(UA u, int blk, int nblk, unsi
         // k = 0 advances in FP64: the arrays hold c - mean, so their k = 0 coefficient stays 0
         // and mean_new = m1(0) mean + m2(0) G(0) / N
         const double mu = *mean;
-        *mean = m1_0 * mu + m2_0 * g0 * u.scale;
+        *((kApart && u.mean_out) ? u.mean_out : mean) = m1_0 * mu + m2_0 * g0 * u.scale;
         c[0] = mk<T>(T(0), T(0));
     }
-    store_line<T, E>(c, sarr, base, ti.es, lm.t, TT, valid);
+    store_line<T, E>(c, sout, base, ti.es, lm.t, TT, valid);
     if (MON) {
         // the state is FFT(c) / N: |FFT(c)|^2 = |S|^2 / scale^2
         double* red = reinterpret_cast<double*>(lds + lds_elems(n, a.TW));

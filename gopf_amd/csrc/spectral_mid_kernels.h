@@ -50,12 +50,33 @@ struct MidL {
     const double* axis;  // the table's part of the line's axis
     int vary;            // that axis: 0 x, 1 y, 2 z
     double fy, fx, fz;   // the fixed components
-    __device__ __forceinline__ double at(int p) const {
+    __device__ __forceinline__ double f2(int p) const {
         const double v = axis[p];
         const double y = (vary == 1) ? v : fy, x = (vary == 0) ? v : fx, z = (vary == 2) ? v : fz;
-        return -(4.0 * 3.14159265358979323846 * 3.14159265358979323846) * (y * y + x * x + z * z);
+        return y * y + x * x + z * z;
+    }
+    __device__ __forceinline__ double at(int p) const {
+        return -(4.0 * 3.14159265358979323846 * 3.14159265358979323846) * f2(p);
     }
 };
+
+// the line of tile line l
+__device__ __forceinline__ MidL mid_line(const KGrid& g, const TileInfo& ti, int l, int& kx) {
+    MidL m;
+    const int bl = ti.b0 + l;
+    const int k0 = ksel(ti.ksrc0, ti.kfix0, ti.ia, bl, 0);
+    const int k1 = ksel(ti.ksrc1, ti.kfix1, ti.ia, bl, 0);
+    const int k2 = ksel(ti.ksrc2, ti.kfix2, ti.ia, bl, 0);
+    double fr[3];
+    ref_freq(g, k0, k1, k2, fr);
+    m.vary = (ti.ksrc0 == 2) ? 0 : (ti.ksrc1 == 2) ? 1 : 2;
+    m.axis = g.ftab + (m.vary == 1 ? 0 : m.vary == 0 ? g.ny : g.ny + g.nx / 2 + 1);
+    m.fy = fr[0];
+    m.fx = fr[1];
+    m.fz = fr[2];
+    kx = k0;
+    return m;
+}
 
 // elements whose operands are in flight together: a divisor of E, bounded so that FP32 keeps
 // four and FP64 two to three waves per SIMD
@@ -98,17 +119,8 @@ __global__ void __launch_bounds__(kMaxBlock) k_mid(MidArgs<T> a) {
     const int op = a.op;
     MidL lap{};
     if (a.need_l) {
-        const int bl = ti.b0 + l;
-        const int k0 = ksel(ti.ksrc0, ti.kfix0, ti.ia, bl, 0);
-        const int k1 = ksel(ti.ksrc1, ti.kfix1, ti.ia, bl, 0);
-        const int k2 = ksel(ti.ksrc2, ti.kfix2, ti.ia, bl, 0);
-        double fr[3];
-        ref_freq(a.g, k0, k1, k2, fr);
-        lap.vary = (ti.ksrc0 == 2) ? 0 : (ti.ksrc1 == 2) ? 1 : 2;
-        lap.axis = a.g.ftab + (lap.vary == 1 ? 0 : lap.vary == 0 ? a.g.ny : a.g.ny + a.g.nx / 2 + 1);
-        lap.fy = fr[0];
-        lap.fx = fr[1];
-        lap.fz = fr[2];
+        int kx;
+        lap = mid_line(a.g, ti, l, kx);
     }
     auto weight = [&](const MidTerm<T>& t, int e) {
         double m = t.coef;
