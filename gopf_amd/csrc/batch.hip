@@ -24,6 +24,7 @@
 #include "../../include/gpf.h"
 #include "batch.h"
 #include "fft_core.h"
+#include "hostcopy.h"
 #include "model.h"
 #include "spectral.h"
 
@@ -46,6 +47,8 @@ struct DBuf {
     }
     void alloc(size_t c) {
         if (p) (void)hipFree(p);
+        p = nullptr;
+        n = 0;
         BCHK(hipMalloc(reinterpret_cast<void**>(&p), (c ? c : 1) * sizeof(T)));
         n = c;
     }
@@ -188,8 +191,12 @@ public:
         BatchClass<T>& c = cls_of(sim);
         const int ls = sim - c.first;
         if (n != (long)c.ny * c.nx) throw BatchError(GPF_EINVAL, "buffer length does not match the sim grid");
-        DBuf<T> tmp(n);
-        DBuf<cpx<T>> tk((size_t)c.ny * (c.nx / 2) + c.ny);
+        // scratch of the largest sim read so far, kept: hipFree waits for the whole device
+        const size_t wantk = (size_t)c.ny * (c.nx / 2) + c.ny;
+        if (gtmp_.n < (size_t)n) gtmp_.alloc(n);
+        if (gtk_.n < wantk) gtk_.alloc(wantk);
+        DBuf<T>& tmp = gtmp_;
+        DBuf<cpx<T>>& tk = gtk_;
         sim_pencils(c, tk.p, tk.p + (long)c.ny * (c.nx / 2), c.S.p + (long)ls * c.ny * (c.nx / 2),
                     c.S.p + c.nmain + (long)ls * c.ny, +1);
         RowC2RArgs<T> a;
@@ -203,16 +210,19 @@ public:
         a.TW = pick_tw(c.nx, 0);
         a.scale = T(1);
         BCHK(launch_rows_c2r<T>(a, st_));
-        std::vector<T> h(n);
         double mean = 0.0;
-        BCHK(hipMemcpyAsync(h.data(), tmp.p, n * sizeof(T), hipMemcpyDeviceToHost, st_));
-        BCHK(hipMemcpyAsync(&mean, c.mean.p + ls, sizeof(double), hipMemcpyDeviceToHost, st_));
-        BCHK(hipStreamSynchronize(st_));
-        if (sizeof(T) != 4) mean = 0.0;
-        for (long j = 0; j < n; ++j) {
-            out[2 * j] = (double)h[j] + mean;
-            out[2 * j + 1] = 0.0;
+        if (sizeof(T) == 4) {
+            BCHK(hipMemcpyAsync(&mean, c.mean.p + ls, sizeof(double), hipMemcpyDeviceToHost, st_));
+            BCHK(hipStreamSynchronize(st_));
         }
+        stage_.download(tmp.p, n * sizeof(T), st_, [&](const char* from, size_t off, size_t len) {
+            const T* h = reinterpret_cast<const T*>(from);
+            double* o = out + 2 * (off / sizeof(T));
+            for (size_t j = 0; j < len / sizeof(T); ++j) {
+                o[2 * j] = (double)h[j] + mean;
+                o[2 * j + 1] = 0.0;
+            }
+        });
     }
 
     void propagate(int nsteps) override {
@@ -629,6 +639,9 @@ private:
     double dt_;
     bool autotune_ = false, tuned_ = false, dirty_ = true;
     hipStream_t st_ = nullptr;
+    HostStage stage_;  // the caller's arrays to and from the device
+    DBuf<T> gtmp_;     // get_field's real and half-transformed scratch
+    DBuf<cpx<T>> gtk_;
     std::vector<std::unique_ptr<BatchClass<T>>> cls_;
     std::vector<std::map<std::string, std::complex<double>>> scalars_;
     int nsims_ = 0, npoly_ = 0;

@@ -39,6 +39,7 @@
 #include "batch.h"
 #include "common.h"
 #include "fft_core.h"
+#include "hostcopy.h"
 #include "io.h"
 #include "reduce.h"
 #include "krylov.h"
@@ -727,6 +728,7 @@ private:
     Buf<double> mean_;          // FP32 fused path: FP64 mean of the field (the arrays hold c - mean)
     bool split_mean_ = false;
     double host_mean();
+    HostStage stage_;           // the caller's arrays to and from the device
     // monitors
     bool mon_ = false;
     std::vector<double> mon_poly_;
@@ -1128,25 +1130,30 @@ void Engine<T>::c2r(const std::vector<const cpx<T>*>& in, const std::vector<T*>&
 template <typename T>
 void Engine<T>::set_field(int idx, const double* in) {
     if (idx < 0 || idx >= nf_) throw Error(GPF_EINVAL, "field index out of range");
-    std::vector<T> h(g_.n);
-    double s = 0.0, c = 0.0;
-    for (long j = 0; j < g_.n; ++j) {
-        const double v = in[2 * j];
-        const double t = s + v;
-        c += (std::fabs(s) >= std::fabs(v)) ? ((s - t) + v) : ((v - t) + s);
-        s = t;
+    double mean = 0.0;
+    if (fp_.ok && split_mean_) {
+        double s = 0.0, c = 0.0;
+        for (long j = 0; j < g_.n; ++j) {
+            const double v = in[2 * j];
+            const double t = s + v;
+            c += (std::fabs(s) >= std::fabs(v)) ? ((s - t) + v) : ((v - t) + s);
+            s = t;
+        }
+        mean = (s + c) / (double)g_.n;
     }
-    const double mean = (fp_.ok && split_mean_) ? (s + c) / (double)g_.n : 0.0;
-    for (long j = 0; j < g_.n; ++j) h[j] = (T)(in[2 * j] - mean);
+    T* dst = fp_.ok ? rscratch(0) : F_[idx].get();
+    stage_.upload(dst, g_.n * sizeof(T), st_, [&](char* to, size_t off, size_t len) {
+        T* h = reinterpret_cast<T*>(to);
+        const double* x = in + 2 * (off / sizeof(T));
+        for (size_t j = 0; j < len / sizeof(T); ++j) h[j] = (T)(x[2 * j] - mean);
+    });
     if (fp_.ok) {
-        T* tmp = rscratch(0);
-        HIPCHK(hipMemcpyAsync(tmp, h.data(), g_.n * sizeof(T), hipMemcpyHostToDevice, st_));
+        T* tmp = dst;
         r2c({tmp}, {S_.get()}, (T)(1.0 / (double)g_.n));
         prime();
         HIPCHK(hipMemcpyAsync(mean_.get(), &mean, sizeof(double), hipMemcpyHostToDevice, st_));
         HIPCHK(hipStreamSynchronize(st_));
     } else {
-        HIPCHK(hipMemcpyAsync(F_[idx].get(), h.data(), g_.n * sizeof(T), hipMemcpyHostToDevice, st_));
         HIPCHK(hipStreamSynchronize(st_));
         kvalid_ = false;
     }
@@ -1155,21 +1162,23 @@ void Engine<T>::set_field(int idx, const double* in) {
 template <typename T>
 void Engine<T>::get_field(int idx, double* out) {
     if (idx < 0 || idx >= nf_) throw Error(GPF_EINVAL, "field index out of range");
-    std::vector<T> h(g_.n);
+    const T* src = F_.empty() ? nullptr : F_[idx].get();
     if (fp_.ok) {
         T* tmp = rscratch(0);
         c2r({S_.get()}, {tmp}, T(1));
-        HIPCHK(hipMemcpyAsync(h.data(), tmp, g_.n * sizeof(T), hipMemcpyDeviceToHost, st_));
-    } else {
-        HIPCHK(hipMemcpyAsync(h.data(), F_[idx].get(), g_.n * sizeof(T), hipMemcpyDeviceToHost, st_));
+        src = tmp;
     }
     HIPCHK(hipStreamSynchronize(st_));
     check_persist();
     const double mean = host_mean();
-    for (long j = 0; j < g_.n; ++j) {
-        out[2 * j] = (double)h[j] + mean;
-        out[2 * j + 1] = 0.0;
-    }
+    stage_.download(src, g_.n * sizeof(T), st_, [&](const char* from, size_t off, size_t len) {
+        const T* h = reinterpret_cast<const T*>(from);
+        double* o = out + 2 * (off / sizeof(T));
+        for (size_t j = 0; j < len / sizeof(T); ++j) {
+            o[2 * j] = (double)h[j] + mean;
+            o[2 * j + 1] = 0.0;
+        }
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -3389,12 +3398,11 @@ public:
     long size() const override { return n_; }
     void exec(double* data, int dir) override {
         ensure();
-        std::vector<cpx<T>> h(n_);
-        for (long i = 0; i < n_; ++i) {
-            h[i].x = (T)data[2 * i];
-            h[i].y = (T)data[2 * i + 1];
-        }
-        HIPCHK(hipMemcpyAsync(d_.get(), h.data(), n_ * sizeof(cpx<T>), hipMemcpyHostToDevice, st_));
+        stage_.upload(d_.get(), n_ * sizeof(cpx<T>), st_, [&](char* to, size_t off, size_t len) {
+            T* h = reinterpret_cast<T*>(to);
+            const double* x = data + off / sizeof(T);
+            for (size_t j = 0; j < len / sizeof(T); ++j) h[j] = (T)x[j];
+        });
         if (nx_ > 1) {
             Seg s;
             s.na = 1; s.nb = (int)(ny_ * nz_); s.sb = nx_; s.es = 1;
@@ -3410,12 +3418,11 @@ public:
             s.na = ny_; s.nb = nx_; s.sa = nx_; s.sb = 1; s.es = (long)nx_ * ny_;
             pass(s, nz_, dir);
         }
-        HIPCHK(hipMemcpyAsync(h.data(), d_.get(), n_ * sizeof(cpx<T>), hipMemcpyDeviceToHost, st_));
-        HIPCHK(hipStreamSynchronize(st_));
-        for (long i = 0; i < n_; ++i) {
-            data[2 * i] = (double)h[i].x;
-            data[2 * i + 1] = (double)h[i].y;
-        }
+        stage_.download(d_.get(), n_ * sizeof(cpx<T>), st_, [&](const char* from, size_t off, size_t len) {
+            const T* h = reinterpret_cast<const T*>(from);
+            double* x = data + off / sizeof(T);
+            for (size_t j = 0; j < len / sizeof(T); ++j) x[j] = (double)h[j];
+        });
     }
 
 private:
@@ -3499,6 +3506,7 @@ private:
     long n_;
     hipStream_t st_ = nullptr;
     Buf<cpx<T>> d_;
+    HostStage stage_;
     std::vector<std::pair<int, Buf<cpx<T>>>> tw_;
     struct Blue {
         int n = 0, dir = 0, m = 0;
