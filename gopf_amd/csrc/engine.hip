@@ -1168,17 +1168,20 @@ void Engine<T>::get_field(int idx, double* out) {
         c2r({S_.get()}, {tmp}, T(1));
         src = tmp;
     }
-    HIPCHK(hipStreamSynchronize(st_));
-    check_persist();
-    const double mean = host_mean();
-    stage_.download(src, g_.n * sizeof(T), st_, [&](const char* from, size_t off, size_t len) {
+    double mean = 0.0;
+    auto ready = [&] {
+        check_persist();
+        mean = host_mean();
+    };
+    auto use = [&](const char* from, size_t off, size_t len) {
         const T* h = reinterpret_cast<const T*>(from);
         double* o = out + 2 * (off / sizeof(T));
         for (size_t j = 0; j < len / sizeof(T); ++j) {
             o[2 * j] = (double)h[j] + mean;
             o[2 * j + 1] = 0.0;
         }
-    });
+    };
+    stage_.download(src, g_.n * sizeof(T), st_, use, ready);
 }
 
 // ---------------------------------------------------------------------------

@@ -29,9 +29,20 @@ public:
     ~HostStage() { release(); }
 
     // use(src, off, len) for every chunk of the bytes at dev, off and len multiples of 16 but at the
-    // end, from several threads at once; returns when all are used
-    template <typename F>
-    void download(const void* dev, size_t bytes, hipStream_t st, F&& use) {
+    // end, from several threads at once; returns when all are used.  ready() runs before the first
+    // use, once the stream's work and the first copy have ended (one wait for both: a wait of its
+    // own cost 7 us of a 32^2 read-back)
+    template <typename F, typename R>
+    void download(const void* dev, size_t bytes, hipStream_t st, F&& use, R&& ready) {
+        if (bytes <= kChunkMin) {
+            if (small_.size() < bytes) wait_small(st), small_.resize(bytes);
+            HIPCHK(hipMemcpyAsync(small_.data(), dev, bytes, hipMemcpyDeviceToHost, st));
+            HIPCHK(hipStreamSynchronize(st));
+            small_busy_ = false;
+            ready();
+            use(static_cast<const char*>(small_.data()), (size_t)0, bytes);
+            return;
+        }
         const Plan p = plan(bytes);
         auto issue = [&](size_t c) {
             const size_t off = c * p.chunk, len = std::min(p.chunk, bytes - off);
@@ -39,6 +50,8 @@ public:
             HIPCHK(hipEventRecord(ev_[p.index(c)], st));
         };
         for (size_t c = 0; c < std::min(p.chunks, (size_t)p.slots); ++c) issue(c);
+        HIPCHK(hipEventSynchronize(ev_[0]));
+        ready();
         run(p, st, [&](size_t c) {
             HIPCHK(hipEventSynchronize(ev_[p.index(c)]));
             const size_t off = c * p.chunk;
@@ -47,10 +60,23 @@ public:
         });
     }
 
+    template <typename F>
+    void download(const void* dev, size_t bytes, hipStream_t st, F&& use) {
+        download(dev, bytes, st, use, [] {});
+    }
+
     // fill(dst, off, len) for every chunk, copied to dev in stream order; returns when every chunk is
     // filled and on its way (the copies end in stream order)
     template <typename F>
     void upload(void* dev, size_t bytes, hipStream_t st, F&& fill) {
+        if (bytes <= kChunkMin) {
+            wait_small(st);
+            if (small_.size() < bytes) small_.resize(bytes);
+            fill(small_.data(), (size_t)0, bytes);
+            small_busy_ = true;
+            HIPCHK(hipMemcpyAsync(dev, small_.data(), bytes, hipMemcpyHostToDevice, st));
+            return;
+        }
         const Plan p = plan(bytes);
         run(p, st, [&](size_t c) {
             const size_t off = c * p.chunk, len = std::min(p.chunk, bytes - off);
@@ -74,6 +100,11 @@ private:
         int workers = 1, slots = 1;
         int index(size_t c) const { return (int)(c % slots); }
     };
+
+    void wait_small(hipStream_t st) {
+        if (small_busy_) HIPCHK(hipStreamSynchronize(st));
+        small_busy_ = false;
+    }
 
     // chunk c belongs to worker c mod workers and slot c mod slots (slots a multiple of workers or
     // one per chunk), so a slot is only ever used by one worker
@@ -156,6 +187,8 @@ private:
         cap_ = 0;
     }
 
+    std::vector<char> small_;  // a field of one chunk: one pageable copy, no pinned memory
+    bool small_busy_ = false;  // an upload may still read it
     char* buf_ = nullptr;
     size_t cap_ = 0;
     std::vector<hipEvent_t> ev_;
