@@ -331,22 +331,20 @@ def c4_traffic(N: int, s: int) -> dict:
     counted once per pass that reads or writes it.  R = a real array (N^3 s bytes), H = a
     half spectrum ((N/2+1) N^2 complex values), K = a per-k table in the field precision
     ((N/2+1) N^2 values of s bytes: the elastic multiplier, and each RK4 stage's factor).
-    Per step: the derived fields' transform (rows with the polynomials inline, y, z) 2R+4H
-    read / 6H written; the elastic term (rows of phi with the indicator inline, y, z; the
-    K(k) multiply; z, y inverse; the fused row pass of H'(phi)(S - 2 e* H(phi)), which reads
-    phi; y, z) 2R+8H+K / 9H; eight RK4 stage passes (conc 13H / 8H, phase 17H / 8H, and the
-    stage factor table, one K per pass); three between-stage syncs (z, y inverse of both
-    fields, the fused row pass, y, z forward of both derived fields) 30H / 30H; the last
-    inverse (z, y, rows) 6H / 4H+2R; the lagged-field copy R / R.
-    FP64 (s = 8) does each stage's update in the fields' first inverse pencil pass: the
-    corrected spectra are neither read back by that pass (8H) nor, before the last stage,
-    written (6H)."""
+    Per step: the derived fields' transform (rows with the polynomials inline, y) 2R+2H read /
+    4H written; the elastic term (rows of phi with the indicator inline, y; the z transforms
+    around the multiply by K(k); y inverse; the fused row pass of H'(phi)(S - 2 e* H(phi)),
+    which reads phi; y, z) 2R+6H+K / 7H; eight middle passes, each the z transform of a field's
+    derived spectrum, its RK4 stage and the inverse z transform (conc 12H / 8H, phase 16H / 8H
+    over the four stages, less the first stage's FINAL and INIT, which are the field's own; a
+    stage factor table, one K per pass) 24H+8K / 16H; three between-stage syncs (y inverse of both
+    fields, the fused row pass, y forward of both derived fields) 18H / 18H; the last inverse
+    (y, rows) 4H / 2H+2R; the lagged-field copy R / R."""
     R = N ** 3 * s
     H = (N // 2 + 1) * N * N * 2 * s
     K = (N // 2 + 1) * N * N * s
-    fused = s == 8
-    rd = 5 * R + (70 if fused else 78) * H + 9 * K
-    wr = 3 * R + (59 if fused else 65) * H
+    rd = 5 * R + 54 * H + 9 * K
+    wr = 3 * R + 47 * H
     return {"read": rd, "write": wr, "total": rd + wr, "per_voxel_step": (rd + wr) / N ** 3}
 
 
