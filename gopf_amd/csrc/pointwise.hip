@@ -7,7 +7,7 @@
 //                 (euler.go:32-38, rk4.go:77-127) and ApplyModalFilter (util.go:125-132)
 //   k_etd_residual  the spectral part of ImplicitEuler's residual (implicitEuler.go:68-94)
 //   k_kgrad       i 2 pi f_d u(k) with f_d = +0.5 zeroed (squareGradientTerm.go:44-50)
-//   k_kelastic    scalar Khachaturyan kernel K(k): force (effectiveForce.go:26-35), 3x3
+//   k_kelastic_table  scalar Khachaturyan kernel K(k): force (effectiveForce.go:26-35), 3x3
 //                 displacement solve (linearElasticity.go:33-63), strains
 //                 (linearElasticity.go:67-83) and the sigma*:eps sum (homoLinElast.go:72-89)
 //                 collapsed by linearity into one multiplier of FFT(H)
