@@ -2506,6 +2506,7 @@ void Engine<T>::etd_mid(const double* x, const double* v, int npt, const double*
         r.nx = g_.nx;
         r.TW = rows_tw(g_.rows, 1);
         HIPCHK(launch_rows_poly(r, st_));
+        half_derived_ = true;
         if (g_.ndim == 3) pencils(lines, {}, 1, -1);
         MidArgs<T> a = mid_args(kMidResidual);
         a.nf = nf_;
@@ -2819,6 +2820,9 @@ void Engine<T>::implicit_step() {
         ++nk_newton_;
     }
     if (!nk_conv_) std::fprintf(stderr, "Warning: Iterative solver did not converge\n");
+    // a constraint's indicator is read from the derived bricks, which an unconverged solve leaves at
+    // the last directional derivative (the sources themselves are needed at the result)
+    if (mid && !nk_conv_ && !vc_state_.empty()) implicit_residual(nx_.get(), nfx_.get());
     // the fields take the solution (implicitEuler.go:205); after a converged check the
     // k-space bricks of the fields are FFT(x) already (the middle pass leaves them unless an
     // equation reads a field's spectrum)

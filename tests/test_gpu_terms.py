@@ -152,6 +152,75 @@ def test_volume_conserving_stepper_propagate_skips_the_update():
     assert np.array_equal(a.Field("phase").real, b.Field("phase").real)
 
 
+def volume_pair(dims, dt):
+    """One field, a polynomial source and a constraint on a derived indicator: every brick is a
+    dense polynomial and there are at most four, so that ImplicitEuler takes its middle pass too."""
+    n = int(np.prod(dims))
+    x = np.meshgrid(*[np.arange(d) for d in dims], indexing="ij")
+    inside = np.all([(xi > 0.3 * d) & (xi < 0.7 * d) for xi, d in zip(x, dims)], axis=0)
+    phase = (0.1 + 0.8 * inside.reshape(-1)) + 0.02 * (np.random.default_rng(12).random(n) - 0.5)
+    pm, om = G.Model(), P.Model()
+    pm.AddField("phase", phase)
+    om.add_field("phase", n)
+    polys = {"WELL_DERIV": [(-0.6, {"phase": 1.0}), (1.8, {"phase": 2.0}), (-1.2, {"phase": 3.0})],
+             "INDICATOR": [(6.0, {"phase": 1.0}), (-6.0, {"phase": 2.0})]}
+    pm.AddScalar("kappa", 0.1)
+    om.add_scalar("kappa", 0.1)
+    for name, poly in polys.items():
+        pm.RegisterPolynomial(name, poly)
+        om.register_polynomial(name, poly)
+    pm.RegisterExplicitTerm("HOLD", G.NewVolumeConservingLP("phase", "INDICATOR", dt, n))
+    om.register_explicit_term("HOLD", P.KIND_VOLCONS, field="phase", indicator="INDICATOR", dt=dt, num_nodes=n)
+    eq = "dphase/dt = WELL_DERIV + kappa*LAP phase + HOLD"
+    pm.AddEquation(eq)
+    om.add_equation(eq)
+    pm.Init()
+    om.init()
+    return pm, om, {"phase": phase.astype(complex)}
+
+
+VOLUME_DIMS = [[16, 16], [9, 20], [10, 10, 10], [7, 7, 7]]
+
+
+@pytest.mark.parametrize("tol,maxiter", [(1e-12, 50), (1e-30, 8)], ids=["converged", "stopped"])
+@pytest.mark.parametrize("dims", VOLUME_DIMS, ids=str)
+def test_volume_conserving_implicit_euler(dims, tol, maxiter):
+    """The multiplier after each step divides by the sum of the indicator over the whole domain at
+    the step's result (volumeConserving.go:31-50); it is nonzero from the third step on.  A tolerance
+    that no iterate meets stops at the same root with the solve unconverged."""
+    dt = 0.1
+    pm, om, init = volume_pair(dims, dt)
+    s = G.Solver(pm, dims, dt, stepper="implicitEuler")
+    s.SetNewtonKrylov(Maxiter=maxiter, Tol=tol)
+    o = ImplicitEulerOracle(om, dims, init, dt, f_tol=1e-12)
+    for _ in range(6):
+        s.Propagate(1)
+        assert s.NewtonStats()["converged"] == (tol > 1e-20)
+        o.step()
+        o.o.on_step_finished()
+    assert o.o.volcons_multiplier() != 0.0
+    assert maxrel(s.Field("phase").real, o.field("phase").real) <= 1e-9
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("dims", VOLUME_DIMS, ids=str)
+@pytest.mark.parametrize("stepper", ["euler", "rk4"])
+def test_volume_conserving_derived_indicator(stepper, dims, precision):
+    """The indicator's integral from a brick that is not transformed along the last axis."""
+    dt, steps = 0.1, 12
+    pm, om, init = volume_pair(dims, dt)
+    s = G.Solver(pm, dims, dt, stepper=stepper, precision=precision)
+    o = OracleSolver(om, dims, init, dt, stepper=stepper)
+    s.Propagate(steps)
+    o.solver_propagate(steps)
+    assert o.volcons_multiplier() != 0.0
+    a, b = s.Field("phase").real, o.field("phase").real
+    if precision == "fp64":
+        assert maxrel(a, b) <= 1e-10
+    else:
+        assert np.linalg.norm(a - b) / np.linalg.norm(b) <= 1e-5
+
+
 HESS_CASES = {
     "2d_diag": ([32, 32], [1.0, 0.0, 0.0, 0.5]),
     "3d_diag": ([16, 16, 16], [1.0, 0.0, 0.0, 0.0, 0.7, 0.0, 0.0, 0.0, 0.4]),
