@@ -281,7 +281,7 @@ static int choose_tw(int n, size_t elem, int min_tw) {
 template <typename F>
 static int fit_tw(int n, size_t elem, int variant, bool strided, long lines, F&& blocks, int min_threads = 0) {
     const int T = fft_threads_per_line(n, variant);
-    const int most = std::max((strided && elem == 16) ? 128 : 256, std::min(2 * T, kMaxBlockThreads));
+    const int most = std::max({(strided && elem == 16) ? 128 : 256, std::min(2 * T, kMaxBlockThreads), min_threads});
     const bool small = T < 64 && (double)lines * T <= (strided ? 4096.0 : 5120.0) * 64.0;
     int best = 1;
     double bc = 1e300;
@@ -614,6 +614,17 @@ private:
     int upd_axis() const { return (g_.ndim == 3) ? upd_axis_ : 1; }
     int other_axis() const { return upd_axis() == 2 ? 1 : 2; }
     int axis_len(int axis) const { return axis == 2 ? g_.nz : g_.ny; }
+    // Threads per block of an untuned pass of `lines` lines of per_line threads with the monitor (0
+    // without it).  One wavefront of the next row pass adds up the blocks' partial sums, 64 at a
+    // time, and folds the series slot with at least 64 threads: blocks of 256 threads unless they
+    // would be fewer than 256 (us a step with blocks of 64 and 128 threads, and of 256: 192^3 FP32
+    // 110.0 and 83.4, FP64 157.0 and 137.8; 256^3 FP64 295 and 273; 128^3 FP32 51.8 and 48.9)
+    int mon_threads(long lines, int per_line) const {
+        if (!mon_) return 0;
+        int t = 256;
+        while (t > 64 && lines * per_line < 256L * t) t /= 2;
+        return t;
+    }
     // lines per block of an untuned row pass over `lines` transform lines
     int rows_tw(long lines, int variant = 0, int min_threads = 0) const {
         return fit_tw(g_.nx, sizeof(cpx<T>), variant, false, lines, [&](int tw) { return (lines + tw - 1) / tw; },
@@ -1355,8 +1366,8 @@ RowFusedArgs<T> Engine<T>::rows_args(cpx<T>* W, double* mean, int tw, int var) {
     ra.g_nyq = W + g_.nmain;
     ra.rows = g_.rows;
     ra.nx = g_.nx;
-    // (the monitor folds the series slot into row blocks of at least 64 threads)
-    ra.TW = tw > 0 ? tw : rows_tw((g_.rows + 1) / 2, var, mon_ ? 64 : 0);
+    const long lines = (g_.rows + 1) / 2;
+    ra.TW = tw > 0 ? tw : rows_tw(lines, var, mon_threads(lines, fft_threads_per_line(g_.nx, var)));
     ra.variant = var;
     ra.c_out = c_out_;
     ra.npoly = (int)fp_.gpoly.size();
@@ -1379,9 +1390,11 @@ PencilUpdateArgs<T> Engine<T>::update_args(cpx<T>* S, cpx<T>* W, double* mean, i
     u.p.seg[0] = (axis == 2) ? seg_z_main(g_) : seg_y_main(g_);
     u.p.seg[1] = (axis == 2) ? seg_z_nyq(g_) : seg_y_nyq(g_);
     u.p.nseg = 2;
+    const long lines = pencil_blocks(u.p.seg, u.p.nseg, 1, nullptr);
     u.p.TW = tw > 0 ? tw
-                    : fit_tw(nu, sizeof(cpx<T>), 1, true, pencil_blocks(u.p.seg, u.p.nseg, 1, nullptr),
-                             [&](int t) { return pencil_blocks(u.p.seg, u.p.nseg, t, nullptr); });
+                    : fit_tw(nu, sizeof(cpx<T>), 1, true, lines,
+                             [&](int t) { return pencil_blocks(u.p.seg, u.p.nseg, t, nullptr); },
+                             mon_threads(lines, fft_threads_per_line(nu, 1)));
     u.g = g_.kg;
     u.dt = dt_;
     u.scale = 1.0 / (double)g_.n;

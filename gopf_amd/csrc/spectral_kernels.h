@@ -1515,9 +1515,13 @@ hipError_t launch_pencil_update_set(const PencilUpdateArgs<T>& u0, int n, hipStr
     return dispatch_size<SET>(n, [&](auto NC) -> hipError_t {
         constexpr int NN = decltype(NC)::value;
         const dim3 g(blocks), b(thr);
-        if (u.mtab[0]) {
-            if (u.egrad_partial) return launch_k(k_pencil_update<T, NN, true, true>, g, b, smem, s, u);
-            return launch_k(k_pencil_update<T, NN, false, true>, g, b, smem, s, u);
+        // FP64 lines of 28 elements per thread spill: from 448 on the monitored pass is slower with the
+        // table (us a step with and without: 112^2 37.4 and 39.4, 224^2 42.5 and 42.6, 448^2 48.8 and
+        // 47.2, 896^2 69.4 and 66.5)
+        constexpr bool kMonTab = sizeof(T) == 4 || LineShape<NN, 1>::E < 28 || NN < 448;
+        if (u.mtab[0] && !u.egrad_partial) return launch_k(k_pencil_update<T, NN, false, true>, g, b, smem, s, u);
+        if constexpr (kMonTab) {
+            if (u.mtab[0]) return launch_k(k_pencil_update<T, NN, true, true>, g, b, smem, s, u);
         }
         if (u.egrad_partial) return launch_k(k_pencil_update<T, NN, true, false>, g, b, smem, s, u);
         return launch_k(k_pencil_update<T, NN, false, false>, g, b, smem, s, u);
