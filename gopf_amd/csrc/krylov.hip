@@ -8,6 +8,8 @@
 // sums folds (k_gs_sweep, k_gs_normalize, k_reduce_rows).  Every sum has a fixed order.
 #include "krylov.h"
 
+#include <algorithm>
+
 namespace gpf {
 
 namespace {
@@ -283,11 +285,13 @@ hipError_t launch_absmax(const double* x, long n, double* partial, double* out, 
     return hipGetLastError();
 }
 
-// at most 256 blocks: every block of the next kernel folds one partial per block and vector
+// Every block of the next kernel folds one partial per block and vector: at most 256 blocks, but
+// for long vectors, whose sweeps are bound by memory (one wavefront per SIMD does not load fast
+// enough), more, with 8 elements per thread, up to 1024 (us a step with at most 256, 512, 1024 and
+// 2048: 128^3 of three fields 9009, 8600, 8431 and 8511, 2048^2 5146, 4640, 4449 and 4602)
 long gs_blocks(long n) {
-    long g = (n + kKrylovThreads - 1) / kKrylovThreads;
-    if (g > 256) g = 256;
-    return g < 1 ? 1 : g;
+    const long most = std::clamp(n / (8L * kKrylovThreads), 256L, 1024L);
+    return std::clamp((n + kKrylovThreads - 1) / kKrylovThreads, 1L, most);
 }
 
 hipError_t launch_gs_dots(const double* V, long ld, int nv, const double* w, long n, double* partial, hipStream_t s) {

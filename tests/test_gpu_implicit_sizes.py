@@ -54,3 +54,28 @@ def test_implicit_sizes(dims, nfields, stencil, restart):
     for f in names:
         ref = o.field(f).real
         assert np.abs(s.Field(f).real - ref).max() <= 1e-9 * np.abs(ref).max(), f
+
+
+def test_long_vectors():
+    """Vectors of more than half a million values take more than 256 reduction blocks: two
+    independent fields of one equation and start, solved together, against one alone (256 blocks)."""
+    dims = [448, 640]
+    n = int(np.prod(dims))
+    x = 0.5 + 0.1 * (np.random.default_rng(8).random(n) - 0.5)
+    got = []
+    for names in (["aaa"], ["aaa", "bbb"]):
+        m = G.Model()
+        for f in names:
+            m.AddField(f, x)
+        for k, v in {"m2": 2.0, "m6": 6.0, "m4": 4.0, "mk": 1.0}.items():
+            m.AddScalar(k, v)
+        for f in names:
+            m.AddEquation(f"d{f}/dt = m2*LAP {f} - m6*LAP {f}^2 + m4*LAP {f}^3 - mk*LAP^2 {f}")
+        m.Init()
+        s = G.Solver(m, dims, 0.1, stepper="implicitEuler")
+        s.SetNewtonKrylov(Tol=1e-12)
+        s.Propagate(2)
+        assert s.NewtonStats()["converged"]
+        got += [s.Field(f).real for f in names]
+    for g in got[1:]:
+        assert np.abs(g - got[0]).max() <= 1e-9 * np.abs(got[0]).max()
