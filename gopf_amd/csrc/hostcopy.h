@@ -30,28 +30,29 @@ public:
 
     // use(src, off, len) for every chunk of the bytes at dev, off and len multiples of 16 but at the
     // end, from several threads at once; returns when all are used.  ready() runs before the first
-    // use, once the stream's work and the first copy have ended (one wait for both: a wait of its
-    // own cost 7 us of a 32^2 read-back)
+    // use, once the stream's work has ended: for one chunk with its copy (a wait of its own cost 7 us
+    // of a 32^2 read-back), for several before any copy, so that it may throw or wait itself
     template <typename F, typename R>
     void download(const void* dev, size_t bytes, hipStream_t st, F&& use, R&& ready) {
         if (bytes <= kChunkMin) {
             if (small_.size() < bytes) wait_small(st), small_.resize(bytes);
+            small_busy_ = true;
             HIPCHK(hipMemcpyAsync(small_.data(), dev, bytes, hipMemcpyDeviceToHost, st));
-            HIPCHK(hipStreamSynchronize(st));
-            small_busy_ = false;
+            wait_small(st);
             ready();
             use(static_cast<const char*>(small_.data()), (size_t)0, bytes);
             return;
         }
+        HIPCHK(hipStreamSynchronize(st));
+        ready();
         const Plan p = plan(bytes);
         auto issue = [&](size_t c) {
             const size_t off = c * p.chunk, len = std::min(p.chunk, bytes - off);
             HIPCHK(hipMemcpyAsync(slot(p, c), static_cast<const char*>(dev) + off, len, hipMemcpyDeviceToHost, st));
             HIPCHK(hipEventRecord(ev_[p.index(c)], st));
+            used_[p.index(c)] = 1;  // should the call end before its use
         };
         for (size_t c = 0; c < std::min(p.chunks, (size_t)p.slots); ++c) issue(c);
-        HIPCHK(hipEventSynchronize(ev_[0]));
-        ready();
         run(p, st, [&](size_t c) {
             HIPCHK(hipEventSynchronize(ev_[p.index(c)]));
             const size_t off = c * p.chunk;
@@ -188,13 +189,13 @@ private:
     }
 
     std::vector<char> small_;  // a field of one chunk: one pageable copy, no pinned memory
-    bool small_busy_ = false;  // an upload may still read it
+    bool small_busy_ = false;  // a copy may still read or write it
     char* buf_ = nullptr;
     size_t cap_ = 0;
     std::vector<hipEvent_t> ev_;
     size_t last_chunk_ = 0;
     int last_slots_ = 0;
-    std::vector<char> used_;  // the slot's event has been recorded by an upload
+    std::vector<char> used_;  // the slot's event has been recorded
 };
 
 }  // namespace gpf

@@ -6,6 +6,9 @@
   and both builds parse the parser-parity corpus, the reference's panicking equations and a
   registered function.  The sanitized run must be clean and print exactly what the plain
   run prints.
+* The staging of whole fields between the caller's arrays and the device (gopf_amd/csrc/hostcopy.h)
+  is built the same two ways against a stand-in runtime (tests/sanitize/hip) whose copies run as
+  late as the waits allow, and must move the right bytes, also after a transfer that failed.
 * The C oracle (oracle/pf_oracle.c) is built with the same sanitizers and the oracle's own CPU
   tests run against it in a child process (libasan preloaded, as Python itself is not
   instrumented).
@@ -62,6 +65,16 @@ def test_equation_compiler_under_asan_ubsan(tmp_path):
     # the corpus ran: every case initialised, and every panic was reported
     assert a.stdout.count("PANIC") == 6
     assert "term 0 kind 0" in a.stdout and "brick CHEMPOT" in a.stdout
+
+
+@pytest.mark.parametrize("flags", [[], SAN], ids=["plain", "sanitized"])
+def test_host_copies(tmp_path, flags):
+    out = str(tmp_path / "hostcopy")
+    subprocess.check_call(["g++", "-std=c++17", "-O1", "-pthread"] + flags +
+                          ["-I", os.path.join(HERE, "sanitize"), "-I", os.path.join(ROOT, "gopf_amd", "csrc"),
+                           os.path.join(HERE, "sanitize", "hostcopy_driver.cpp"), "-o", out])
+    r = subprocess.run([out], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout + r.stderr
 
 
 def test_oracle_under_asan_ubsan(tmp_path):
