@@ -3,8 +3,8 @@
 // A pageable hipMemcpy of a field goes through the runtime's own staging on one thread, the
 // conversion to or from the caller's complex128 is another pass over a temporary, and a fresh
 // array's page faults are taken one by one (256^3 FP32 read back in about 22 ms, now 4.4;
-// the wire needs 1.3).  HostStage copies chunks into pinned memory while a few threads convert the
-// chunks that have arrived.  The pinned memory belongs to the object (at most kWorkers kSlots
+// the wire needs 1.3).  HostStage copies the chunks of a large field into pinned memory while a few
+// threads convert the chunks that have arrived.  The pinned memory belongs to the object (at most kWorkers kSlots
 // chunks) and is freed with it; one call at a time per object, as for every handle.
 #pragma once
 
@@ -15,6 +15,7 @@
 #include <mutex>
 #include <system_error>
 #include <thread>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -22,6 +23,10 @@
 namespace gpf {
 
 class HostStage {
+    struct Nothing {
+        void operator()() const {}
+    };
+
 public:
     HostStage() = default;
     HostStage(const HostStage&) = delete;
@@ -30,11 +35,11 @@ public:
 
     // use(src, off, len) for every chunk of the bytes at dev, off and len multiples of 16 but at the
     // end, from several threads at once; returns when all are used.  ready() runs before the first
-    // use, once the stream's work has ended: for one chunk with its copy (a wait of its own cost 7 us
-    // of a 32^2 read-back), for several before any copy, so that it may throw or wait itself
+    // use, once the stream's work has ended: for one copy with it (a wait of its own cost 7 us of a
+    // 32^2 read-back), for chunks before the first of them, so that it may throw or wait itself
     template <typename F, typename R>
     void download(const void* dev, size_t bytes, hipStream_t st, F&& use, R&& ready) {
-        if (bytes <= kChunkMin) {
+        if (bytes <= kDirect) {
             if (small_.size() < bytes) wait_small(st), small_.resize(bytes);
             small_busy_ = true;
             HIPCHK(hipMemcpyAsync(small_.data(), dev, bytes, hipMemcpyDeviceToHost, st));
@@ -43,8 +48,10 @@ public:
             use(static_cast<const char*>(small_.data()), (size_t)0, bytes);
             return;
         }
-        HIPCHK(hipStreamSynchronize(st));
-        ready();
+        if constexpr (!std::is_same<std::decay_t<R>, Nothing>::value) {
+            HIPCHK(hipStreamSynchronize(st));
+            ready();
+        }
         const Plan p = plan(bytes);
         auto issue = [&](size_t c) {
             const size_t off = c * p.chunk, len = std::min(p.chunk, bytes - off);
@@ -63,14 +70,14 @@ public:
 
     template <typename F>
     void download(const void* dev, size_t bytes, hipStream_t st, F&& use) {
-        download(dev, bytes, st, use, [] {});
+        download(dev, bytes, st, use, Nothing{});
     }
 
     // fill(dst, off, len) for every chunk, copied to dev in stream order; returns when every chunk is
     // filled and on its way (the copies end in stream order)
     template <typename F>
     void upload(void* dev, size_t bytes, hipStream_t st, F&& fill) {
-        if (bytes <= kChunkMin) {
+        if (bytes <= kDirect) {
             wait_small(st);
             if (small_.size() < bytes) small_.resize(bytes);
             fill(small_.data(), (size_t)0, bytes);
@@ -91,10 +98,15 @@ public:
     }
 
 private:
-    // chunks of 1 MB against 512 KB: 128^3 complex128 transform 2.4 against 3.2 ms, 256^3 FP32 field
-    // 4.4 against 4.8 ms (eight threads; 5.8 ms with four, 4.0 with twelve); 256 KB against 1 MB for
-    // a field of 1 MB: 0.42 against 0.52 ms
-    static constexpr size_t kChunkMin = (size_t)256 << 10, kChunkMax = (size_t)1 << 20;
+    // Starting a thread costs 20 to 50 us: one thread per MB, and up to kDirect one pageable copy (us
+    // with one copy, a thread per MB, eight threads from 256 KB on; arrays already mapped, then fresh
+    // ones: complex128 transform of 192^2 96, 184, 158; 320^2 250, 229, 338; 512^2 594, 467, 705; FP32
+    // field of 512^2 182, 213, 288 and 282, 267, 331; 640^2 253, 251, 441 and 680, 418, 487; 1024^2
+    // 582, 464, 834 and 1550, 761, 808).  Threads kept waiting between the calls took longer to wake
+    // than new ones to start (192^2 transform 496 us).
+    // Chunks of 1 MB against 512 KB: 128^3 complex128 transform 2.4 against 3.2 ms, 256^3 FP32 field
+    // 4.4 against 4.8 ms (eight threads; 5.8 ms with four, 4.0 with twelve).
+    static constexpr size_t kDirect = (size_t)1280 << 10, kChunkMax = (size_t)1 << 20;
     static constexpr int kWorkers = 8, kSlots = 2;
     struct Plan {
         size_t chunk = 0, chunks = 0;
@@ -111,11 +123,10 @@ private:
     // one per chunk), so a slot is only ever used by one worker
     Plan plan(size_t bytes) {
         Plan p;
-        p.chunk = std::clamp(bytes / (kWorkers * kSlots), kChunkMin, kChunkMax);
-        p.chunk = (std::min(p.chunk, std::max<size_t>(bytes, 1)) + 4095) / 4096 * 4096;
-        p.chunks = std::max<size_t>((bytes + p.chunk - 1) / p.chunk, 1);
         const int cores = std::max(1, (int)std::thread::hardware_concurrency());
-        p.workers = (int)std::min<size_t>({(size_t)kWorkers, (size_t)cores, p.chunks});
+        p.workers = (int)std::clamp<size_t>(bytes >> 20, 2, std::min(kWorkers, std::max(cores, 2)));
+        p.chunk = (std::min(bytes / (p.workers * kSlots), kChunkMax) + 4095) / 4096 * 4096;
+        p.chunks = (bytes + p.chunk - 1) / p.chunk;
         p.slots = (int)std::min<size_t>((size_t)p.workers * kSlots, p.chunks);
         if (p.slots % p.workers) p.slots = p.workers;
         const size_t want = p.chunk * p.slots;
@@ -188,7 +199,7 @@ private:
         cap_ = 0;
     }
 
-    std::vector<char> small_;  // a field of one chunk: one pageable copy, no pinned memory
+    std::vector<char> small_;  // the host's side of one pageable copy
     bool small_busy_ = false;  // a copy may still read or write it
     char* buf_ = nullptr;
     size_t cap_ = 0;

@@ -12,6 +12,7 @@ using gpf::HostStage;
 using Bytes = std::vector<char>;
 
 static int bad = 0;
+static const size_t kDirect = 1280u << 10;  // HostStage's line between one copy and chunks
 
 static Bytes pattern(size_t n, unsigned seed) {
     Bytes b(n);
@@ -38,7 +39,7 @@ static void check(bool ok, const char* what, size_t n) {
 }
 
 int main() {
-    const size_t sizes[] = {1, 4096, 300000, 1u << 20, (4608u << 10), (4608u << 10) + 16, 5000000, 9000016, 40000000};
+    const size_t sizes[] = {1, 4096, 300000, kDirect, kDirect + 16, 3u << 20, 5000000, 9000016, 40000000};
     HostStage h;  // one object over all sizes: its buffers grow and its slots change
     FakeStream st;
     unsigned seed = 1;
@@ -66,7 +67,7 @@ int main() {
                 if ((kind & 1) == 0) {
                     o.download(dev.data(), n, &st, use, [] { throw std::runtime_error("not valid"); });
                 } else {
-                    st.fail_after = n > (4608u << 10) ? 3 : 0;
+                    st.fail_after = n > kDirect ? 3 : 0;
                     o.download(dev.data(), n, &st, use);
                 }
             } catch (const std::exception&) {
