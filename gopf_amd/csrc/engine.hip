@@ -580,7 +580,7 @@ private:
     // step), and m1(0), m2(0)
     Buf<cpx<T>> ptab_;
     Buf<double> pm0_;
-    bool ptab_ok_ = false;
+    int ptab_axis_ = 0;  // the update axis whose pass's arithmetic the table follows (0: not filled)
     void update_table(PencilUpdateArgs<T>& u);
     bool table_pays() const;
     int* pfail_ = nullptr;      // mapped host flag set by a failed device-wide barrier
@@ -1421,15 +1421,16 @@ bool Engine<T>::table_pays() const {
     return (size_t)g_.nk * sizeof(cpx<T>) <= (size_t)(g_.ndim == 3 ? 40 : 12) << 20;
 }
 
-// fills the table at its first use and lets u read it; never within a graph capture, which a step's
+// fills the table at its first use, and again for another update axis (whose pass sums a frequency's
+// squares in another order), and lets u read it; never within a graph capture, which a step's
 // preparation (prepare_fused) precedes
 template <typename T>
 void Engine<T>::update_table(PencilUpdateArgs<T>& u) {
     if (!ptab_.get()) ptab_.alloc(g_.nk);
     if (!pm0_.get()) pm0_.alloc(2);
-    if (!ptab_ok_) {
-        HIPCHK(launch_update_mult_table<T>(u, g_.ndim == 3 ? upd_axis() : 1, g_.nmain, g_.nk, ptab_.get(), pm0_.get(), st_));
-        ptab_ok_ = true;
+    if (ptab_axis_ != upd_axis()) {
+        HIPCHK(launch_update_mult_table<T>(u, upd_axis(), g_.nmain, g_.nk, ptab_.get(), pm0_.get(), st_));
+        ptab_axis_ = upd_axis();
     }
     u.mtab[0] = ptab_.get();
     u.mtab[1] = ptab_.get() + g_.nmain;
@@ -1566,7 +1567,8 @@ void Engine<T>::set_filter(const double* table) {
     if (table && stepper_ == GPF_SDD) throw Error(GPF_EINVAL, "SDD: Does not support modal filters");
     HIPCHK(hipStreamSynchronize(st_));
     drop_graph();
-    stab_ok_ = etab_ok_ = ptab_ok_ = false;
+    stab_ok_ = etab_ok_ = false;
+    ptab_axis_ = 0;
     if (!table) {
         has_filter_ = false;
         return;
@@ -1631,7 +1633,7 @@ void Engine<T>::drop_graph() {
 
 template <typename T>
 void Engine<T>::prepare_fused(long upcoming) {
-    if (!ptab_ok_ && table_pays()) (void)update_args(S_.get(), W_.get(), mean_.get(), tw_pu_);
+    if (ptab_axis_ != upd_axis() && table_pays()) (void)update_args(S_.get(), W_.get(), mean_.get(), tw_pu_);
     if (!mon_) return;
     const long nblk_a = rows_fused_blocks(g_.rows, rows_args(W_.get(), mean_.get(), tw_rows_, rows_var_).TW);
     PencilUpdateArgs<T> u = update_args(S_.get(), W_.get(), mean_.get(), tw_pu_);
