@@ -76,13 +76,6 @@ int pick_tw(int n, int variant) {
     return tw;
 }
 
-// a block of tw lines fits: threads, and LDS for the exchange lines, the row pass's copy of
-// the twiddle table and the monitor's partial sums (160 KiB per workgroup on gfx950)
-bool tw_ok(int n, int tw, size_t elem, int variant) {
-    const size_t lds = ((size_t)(n + n / 16 + 1) * (tw + 1) + n) * elem + (size_t)kMaxBlockThreads * sizeof(double);
-    return tw * fft_threads_per_line(n, variant) <= kMaxBlockThreads && lds <= 160 * 1024;
-}
-
 }  // namespace
 
 // one size class: nsim sims of ny x nx
@@ -262,12 +255,17 @@ public:
         const int nc = (int)cls_.size();
         if (n != 3 * nc + 1) throw BatchError(GPF_EINVAL, "a batch layout has 3 values per class and 1 more");
         if (dirty_) compile();
+        std::vector<int> tr(nc), tu(nc);
         for (int k = 0; k < nc; ++k) {
             BatchClass<T>& c = *cls_[k];
-            const int tr = v[3 * k], tu = v[3 * k + 1], var = v[3 * k + 2];
-            auto pow2 = [](int x) { return x >= 1 && (x & (x - 1)) == 0; };
-            if (!pow2(tr) || !pow2(tu) || (var != 0 && var != 1) || !tw_ok(c.nx, tr, sizeof(cpx<T>), var) ||
-                !tw_ok(c.ny, tu, sizeof(cpx<T>), 1))
+            const int var = v[3 * k + 2];
+            auto lines = [](int len, int tw, int vr) {
+                const bool pow2 = tw >= 1 && (tw & (tw - 1)) == 0;
+                return pow2 && (vr == 0 || vr == 1) ? stored_layout_lines(len, tw, sizeof(cpx<T>), vr) : 0;
+            };
+            tr[k] = lines(c.nx, v[3 * k], var);
+            tu[k] = lines(c.ny, v[3 * k + 1], 1);
+            if (!tr[k] || !tu[k])
                 throw BatchError(GPF_EINVAL, "batch layout not admissible for class " + std::to_string(k));
         }
         const int th = v[3 * nc];
@@ -275,8 +273,8 @@ public:
             throw BatchError(GPF_EINVAL, "grouped launches need power-of-two sides 64..1024 and 128, 256 or 512 threads");
         BCHK(hipStreamSynchronize(st_));
         for (int k = 0; k < nc; ++k) {
-            cls_[k]->tw_rows = v[3 * k];
-            cls_[k]->tw_upd = v[3 * k + 1];
+            cls_[k]->tw_rows = tr[k];
+            cls_[k]->tw_upd = tu[k];
             cls_[k]->rows_var = v[3 * k + 2];
         }
         grouped_ = false;
@@ -475,7 +473,7 @@ private:
             const int tr = threads / fft_threads_per_line(c.nx, c.rows_var);
             const int tu = threads / fft_threads_per_line(c.ny, 1);
             if (tr < 1 || tu < 1 || tr * fft_threads_per_line(c.nx, c.rows_var) != threads ||
-                tu * fft_threads_per_line(c.ny, 1) != threads || !tw_ok(c.nx, tr, el, c.rows_var) || !tw_ok(c.ny, tu, el, 1))
+                tu * fft_threads_per_line(c.ny, 1) != threads || !lines_fit(c.nx, tr, el, c.rows_var) || !lines_fit(c.ny, tu, el, 1))
                 return false;
             ra[k] = rows_args(c, W[k], mu[k], tr, c.rows_var);
             ua[k] = upd_args(c, S[k], W[k], mu[k], tu);
@@ -560,13 +558,13 @@ private:
             float best = 1e30f;
             for (int var = 0; var < 2; ++var)
                 for (int tw : cand) {
-                    if (!tw_ok(c.nx, tw, sizeof(cpx<T>), var)) continue;
+                    if (!lines_fit(c.nx, tw, sizeof(cpx<T>), var)) continue;
                     const float t = time_it([&] { BCHK(launch_rows_fused<T>(rows_args(c, W.p, mu.p, tw, var), st_)); });
                     if (t < best) { best = t; c.tw_rows = tw; c.rows_var = var; }
                 }
             best = 1e30f;
             for (int tw : cand) {
-                if (!tw_ok(c.ny, tw, sizeof(cpx<T>), 1)) continue;
+                if (!lines_fit(c.ny, tw, sizeof(cpx<T>), 1)) continue;
                 const float t = time_it([&] { BCHK(launch_pencil_update<T>(upd_args(c, S.p, W.p, mu.p, tw), c.ny, st_)); });
                 if (t < best) { best = t; c.tw_upd = tw; }
             }

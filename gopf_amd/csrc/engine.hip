@@ -247,14 +247,6 @@ struct Geometry {
     }
 };
 
-// a block of tw lines fits: threads, and LDS for the exchange lines, the row pass's copy of
-// the twiddle table and the monitor's FP64 partial sums (160 KiB per workgroup on gfx950)
-static bool tw_fits(int n, int tw, size_t elem, int variant = 0) {
-    const int T = fft_threads_per_line(n, variant);
-    const size_t lds = ((size_t)(n + n / 16 + 1) * (tw + 1) + n) * elem + (size_t)kMaxBlockThreads * sizeof(double);
-    return tw * T <= kMaxBlockThreads && lds <= 160 * 1024;
-}
-
 // lines per block of the stand-alone transforms: about 256 threads, at least min_tw lines
 static int choose_tw(int n, size_t elem, int min_tw) {
     const int T = fft_threads_per_line(n, 0);
@@ -1494,7 +1486,7 @@ void Engine<T>::autotune() {
         int best = 0;
         float bt = 1e30f;
         for (int tw : cand) {
-            if (!tw_fits(n, tw, sizeof(cpx<T>), variant)) continue;
+            if (!lines_fit(n, tw, sizeof(cpx<T>), variant)) continue;
             const float t = time_it([&] { launch_with(tw); });
             if (t < bt) { bt = t; best = tw; }
         }
@@ -1505,7 +1497,7 @@ void Engine<T>::autotune() {
         float bt = 1e30f;
         for (int var = 0; var < 2; ++var)
             for (int tw : cand) {
-                if (!tw_fits(g_.nx, tw, sizeof(cpx<T>), var)) continue;
+                if (!lines_fit(g_.nx, tw, sizeof(cpx<T>), var)) continue;
                 const float t = time_it([&] { HIPCHK(launch_rows_fused<T>(rows_args(Wb.get(), mu.get(), tw, var), st_)); });
                 if (t < bt) { bt = t; tw_rows_ = tw; rows_var_ = var; }
             }
@@ -1527,7 +1519,7 @@ void Engine<T>::autotune() {
                 for (int var = 0; var < 2; ++var)
                     for (int lpt = 1; lpt <= (sizeof(T) == 4 ? 2 : 1); ++lpt)
                         for (int tw : cand) {
-                            if (!tw_fits(no, tw, sizeof(cpx<T>), var)) continue;
+                            if (!lines_fit(no, tw, sizeof(cpx<T>), var)) continue;
                             const float t = time_it([&] { pencils_tw({Wb.get()}, other_axis(), dir, tw, lpt, var); });
                             if (t < bt) { bt = t; tw_out = tw; lpt_out = lpt; var_out = var; }
                         }
@@ -1596,23 +1588,29 @@ void Engine<T>::set_tuning(const int* v, int n) {
     const int other = (axis == 2) ? 1 : 2;
     const int nu = axis == 2 ? g_.nz : g_.ny, no = other == 2 ? g_.nz : g_.ny;
     const size_t el = sizeof(cpx<T>);
-    auto ok_tw = [](int tw) { return tw == 4 || tw == 8 || tw == 16 || tw == 32 || tw == 64; };
+    // the lines per block, or 0: not admissible
+    auto lines = [&](int len, int tw, int var) {
+        const bool listed = tw == 4 || tw == 8 || tw == 16 || tw == 32 || tw == 64;
+        return listed && (var == 0 || var == 1) ? stored_layout_lines(len, tw, el, var) : 0;
+    };
     const int rows_var = v[5], lpf = v[6], lpi = v[7], vpf = v[8], vpi = v[9];
-    bool ok = ok_tw(v[0]) && ok_tw(v[2]) && (rows_var == 0 || rows_var == 1) && tw_fits(g_.nx, v[0], el, rows_var) &&
-              tw_fits(nu, v[2], el, 1);
+    const int rows = lines(g_.nx, v[0], rows_var), upd = lines(nu, v[2], 1);
+    int fwd = v[1], inv = v[3];
+    bool ok = rows && upd;
     if (g_.ndim == 3) {
-        ok = ok && ok_tw(v[3]) && (vpi == 0 || vpi == 1) && (lpi == 1 || (lpi == 2 && sizeof(T) == 4)) &&
-             tw_fits(no, v[3], el, vpi);
-        if (fp_.has_src)
-            ok = ok && ok_tw(v[1]) && (vpf == 0 || vpf == 1) && (lpf == 1 || (lpf == 2 && sizeof(T) == 4)) &&
-                 tw_fits(no, v[1], el, vpf);
+        inv = lines(no, v[3], vpi);
+        ok = ok && inv && (lpi == 1 || (lpi == 2 && sizeof(T) == 4));
+        if (fp_.has_src) {
+            fwd = lines(no, v[1], vpf);
+            ok = ok && fwd && (lpf == 1 || (lpf == 2 && sizeof(T) == 4));
+        }
     }
     if (!ok) throw Error(GPF_EINVAL, "launch layout not admissible for this grid and precision");
     HIPCHK(hipStreamSynchronize(st_));
-    tw_rows_ = v[0];
-    tw_pf_ = v[1];
-    tw_pu_ = v[2];
-    tw_pi_ = v[3];
+    tw_rows_ = rows;
+    tw_pf_ = fwd;
+    tw_pu_ = upd;
+    tw_pi_ = inv;
     upd_axis_ = axis;
     rows_var_ = rows_var;
     lpt_pf_ = lpf;
@@ -1855,7 +1853,7 @@ void Engine<T>::set_persistent(int mode, int threads) {
         throw Error(GPF_EINVAL, "threads per block of the persistent step: 0 (64), 64, 128, 256 or 512");
     if (threads > 0 && g_.ndim == 2 && persist_side(g_.nx) && g_.nx == g_.ny) {
         const int t1 = fft_threads_per_line(g_.nx, 1);
-        if (threads < t1 || !tw_fits(g_.nx, threads / t1, sizeof(cpx<T>), 1))
+        if (threads < t1 || !lines_fit(g_.nx, threads / t1, sizeof(cpx<T>), 1))
             throw Error(GPF_EINVAL, "threads per block not admissible for this grid's persistent step");
     }
     HIPCHK(hipStreamSynchronize(st_));
@@ -1872,7 +1870,7 @@ void Engine<T>::build_persist() {
     const int t1 = fft_threads_per_line(n, 1);
     const int thr = persist_threads_ > 0 ? persist_threads_ : std::max(64, t1);
     const int tw = thr / t1;
-    if (tw < 1 || tw * t1 != thr || !tw_fits(n, tw, sizeof(cpx<T>), 1))
+    if (tw < 1 || tw * t1 != thr || !lines_fit(n, tw, sizeof(cpx<T>), 1))
         throw Error(GPF_EINVAL, "persistent step: no admissible block for this grid");
     PersistPlan<T> P;
     RowFusedArgs<T> ra = rows_args(W_.get(), mean_.get(), tw, 1);

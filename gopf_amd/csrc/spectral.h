@@ -327,6 +327,14 @@ template <typename T> hipError_t launch_rows_fused(const RowFusedArgs<T>& a, hip
 bool fft_size_supported(int n);      // sizes with a device transform
 bool fft_size_fast(int n);           // sizes with a compiled Stockham schedule
 int fft_threads_per_line(int n, int variant = 0);  // threads per line (variant 1: the update pass)
+// a block of tw lines fits: threads, and LDS for the exchange lines, the row pass's copy of
+// the twiddle table and the monitor's FP64 partial sums (160 KiB per workgroup on gfx950)
+bool lines_fit(int n, int tw, size_t elem, int variant);
+// Lines per block for the tw of a stored launch layout, 0 where it is not admissible.  The lengths
+// 24 and 96 to 768 = 2^a 3 (plain schedule) and 100, 200, 500 and 1000 once had up to four times
+// fewer threads per line: a layout kept from then that fitted then gets the most lines that fit now,
+// halved from tw.
+int stored_layout_lines(int n, int tw, size_t elem, int variant);
 
 // blocks a launch uses (for sizing per-block partial-sum buffers)
 long rows_blocks(long rows, int TW);

@@ -33,6 +33,23 @@ bool fft_size_supported(int n) { return fft_size_fast(n) || (n >= 1 && n <= 64);
 
 int fft_threads_per_line(int n, int variant) { return threads_per_line(n, variant); }
 
+static bool block_fits(int n, int tw, size_t elem, int per_line) {
+    const size_t lds = ((size_t)(n + n / 16 + 1) * (tw + 1) + n) * elem + (size_t)kMaxBlockThreads * sizeof(double);
+    return tw * per_line <= kMaxBlockThreads && lds <= 160 * 1024;
+}
+
+bool lines_fit(int n, int tw, size_t elem, int variant) { return block_fits(n, tw, elem, threads_per_line(n, variant)); }
+
+int stored_layout_lines(int n, int tw, size_t elem, int variant) {
+    if (lines_fit(n, tw, elem, variant)) return tw;
+    const bool three = variant == 0 && (n == 24 || n == 96 || n == 192 || n == 384);
+    const bool five = n == 100 || n == 200 || n == 500 || n == 1000;
+    const int then = three ? n / 24 : (n == 768 && variant == 0) ? 16 : five ? n / 20 : 0;
+    if (then == 0 || !block_fits(n, tw, elem, then)) return 0;
+    while (tw > 1 && !lines_fit(n, tw, elem, variant)) tw /= 2;
+    return tw;
+}
+
 long rows_blocks(long rows, int TW) { return (rows + TW - 1) / TW; }
 long rows_fused_blocks(long rows, int TW) { return ((rows + 1) / 2 + TW - 1) / TW; }
 
