@@ -435,6 +435,7 @@ __device__ __forceinline__ void update_multipliers(const PencilUpdateArgs<T>& u,
 template <typename T, int N, bool MON, typename UA = PencilUpdateArgs<T>, bool EARLY = false, bool MT = false>
 __device__ __forceinline__ void pencil_update_body(UA u, int blk, int nblk, unsigned char* smem) {
     cpx<T>* lds = reinterpret_cast<cpx<T>*>(smem);
+    static_assert(MT || !EARLY, "a line loaded early needs the tabulated multipliers");
     constexpr int V = 1;  // low-register schedule: two lines and the multipliers stay in registers
     constexpr int E = LineShape<N, V>::E;
     const PencilArgs<T>& a = u.p;
@@ -554,19 +555,24 @@ __device__ __forceinline__ void pencil_update_body(UA u, int blk, int nblk, unsi
             }
         }
     } else {
-        // the chunks' expressions written out: with a call of `update` here the persistent step's
-        // kernel is compiled to other instructions (1000 steps of FP64 128^2 with the energy series,
-        // fresh processes in turn: 13.02 against 12.83 ms; on another card 13.28 against 12.94)
         if constexpr (!EARLY) load_line<T, E>(c, sarr, base, ti.es, lm.t, TT, valid);
+        if constexpr (kApart || !EARLY) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const cpx<T> cv = c[e];
-            if (MON && valid) {
-                const double fv = wrapk(lm.t + TT * e, nv) * invv;
-                eg += wk * 4.0 * kPi * kPi * (fixed2 + fv * fv) *
-                      ((double)cv.x * (double)cv.x + (double)cv.y * (double)cv.y);
+            for (int e = 0; e < E; ++e) update(e, c[e], s1a[e], gs[e]);
+        } else {
+            // the same written out: with the call the persistent step's kernel is compiled to other
+            // instructions (1000 steps of FP64 128^2 with the energy series, fresh processes in turn:
+            // 13.02 against 12.83 ms; on another card 13.28 against 12.94)
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const cpx<T> cv = c[e];
+                if (MON && valid) {
+                    const double fv = wrapk(lm.t + TT * e, nv) * invv;
+                    eg += wk * 4.0 * kPi * kPi * (fixed2 + fv * fv) *
+                          ((double)cv.x * (double)cv.x + (double)cv.y * (double)cv.y);
+                }
+                c[e] = mk<T>(cv.x + (s1a[e] * cv.x + gs[e].x), cv.y + (s1a[e] * cv.y + gs[e].y));
             }
-            c[e] = mk<T>(cv.x + (s1a[e] * cv.x + gs[e].x), cv.y + (s1a[e] * cv.y + gs[e].y));
         }
     }
     if (has_k0) {
