@@ -98,15 +98,17 @@ public:
     }
 
 private:
-    // Starting a thread costs 20 to 50 us: one thread per MB, and up to kDirect one pageable copy (us
-    // with one copy, a thread per MB, eight threads from 256 KB on; arrays already mapped, then fresh
-    // ones: complex128 transform of 192^2 96, 184, 158; 320^2 250, 229, 338; 512^2 594, 467, 705; FP32
-    // field of 512^2 182, 213, 288 and 282, 267, 331; 640^2 253, 251, 441 and 680, 418, 487; 1024^2
-    // 582, 464, 834 and 1550, 761, 808).  Threads kept waiting between the calls took longer to wake
-    // than new ones to start (192^2 transform 496 us).
+    // Starting a thread costs 20 to 50 us, and about 250 more where the host did something else
+    // between the calls: one thread per MB, and up to kDirect one pageable copy, from where the
+    // slower of these starts still costs less (us with one copy; a thread per MB, and the same after
+    // a pause; eight threads from 256 KB on, after pauses 50 to 150 more: complex128 transform in FP32
+    // of 512^2, 2 MB, 369; 257 and 503; 421; FP64 of 512^2, 4 MB, 594; 475 and 554; 705).  FP32 field
+    // of 1024^2, 4 MB, into a mapped array and a fresh one: 582 and 1550; 464 and 761; 834 and 808.
+    // Threads kept waiting between the calls took longer to wake than new ones to start (192^2
+    // transform 496 us, one copy 96).
     // Chunks of 1 MB against 512 KB: 128^3 complex128 transform 2.4 against 3.2 ms, 256^3 FP32 field
     // 4.4 against 4.8 ms (eight threads; 5.8 ms with four, 4.0 with twelve).
-    static constexpr size_t kDirect = (size_t)1280 << 10, kChunkMax = (size_t)1 << 20;
+    static constexpr size_t kDirect = (size_t)3584 << 10, kChunkMax = (size_t)1 << 20;
     static constexpr int kWorkers = 8, kSlots = 2;
     struct Plan {
         size_t chunk = 0, chunks = 0;

@@ -12,7 +12,7 @@ using gpf::HostStage;
 using Bytes = std::vector<char>;
 
 static int bad = 0;
-static const size_t kDirect = 1280u << 10;  // HostStage's line between one copy and chunks
+static const size_t kDirect = 3584u << 10;  // HostStage's line between one copy and chunks
 
 static Bytes pattern(size_t n, unsigned seed) {
     Bytes b(n);
@@ -39,7 +39,7 @@ static void check(bool ok, const char* what, size_t n) {
 }
 
 int main() {
-    const size_t sizes[] = {1, 4096, 300000, kDirect, kDirect + 16, 3u << 20, 5000000, 9000016, 40000000};
+    const size_t sizes[] = {1, 4096, 300000, kDirect, kDirect + 16, 4u << 20, 5000000, 9000016, 40000000};
     HostStage h;  // one object over all sizes: its buffers grow and its slots change
     FakeStream st;
     unsigned seed = 1;
