@@ -203,16 +203,14 @@ public:
         a.TW = pick_tw(c.nx, 0);
         a.scale = T(1);
         BCHK(launch_rows_c2r<T>(a, st_));
-        double mean = 0.0;
-        if (sizeof(T) == 4) {
-            BCHK(hipMemcpyAsync(&mean, c.mean.p + ls, sizeof(double), hipMemcpyDeviceToHost, st_));
-            BCHK(hipStreamSynchronize(st_));
-        }
+        // in stream order before the field, which is waited for: no wait of its own
+        gmean_ = 0.0;
+        if (sizeof(T) == 4) BCHK(hipMemcpyAsync(&gmean_, c.mean.p + ls, sizeof(double), hipMemcpyDeviceToHost, st_));
         stage_.download(tmp.p, n * sizeof(T), st_, [&](const char* from, size_t off, size_t len) {
             const T* h = reinterpret_cast<const T*>(from);
             double* o = out + 2 * (off / sizeof(T));
             for (size_t j = 0; j < len / sizeof(T); ++j) {
-                o[2 * j] = (double)h[j] + mean;
+                o[2 * j] = (double)h[j] + gmean_;
                 o[2 * j + 1] = 0.0;
             }
         });
@@ -640,6 +638,7 @@ private:
     HostStage stage_;  // the caller's arrays to and from the device
     DBuf<T> gtmp_;     // get_field's real and half-transformed scratch
     DBuf<cpx<T>> gtk_;
+    double gmean_ = 0.0;  // and the mean of an FP32 sim
     std::vector<std::unique_ptr<BatchClass<T>>> cls_;
     std::vector<std::map<std::string, std::complex<double>>> scalars_;
     int nsims_ = 0, npoly_ = 0;
