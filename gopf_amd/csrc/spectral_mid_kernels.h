@@ -12,8 +12,8 @@ namespace {
 
 // Element access by byte offset from a uniform base: one offset register per element serves all
 // arrays, where 64-bit element indexes cost two registers per element and array.  An array
-// whose lines are shorter than kMidLong is below 4 GiB (800^3 in FP64: 4.1e9 bytes), so its
-// offsets have 32 bits.
+// whose lines are shorter than kMidLong is below 4 GiB, so its offsets have 32 bits: 3D domains are
+// cubes (the largest length before it, 800^3 in FP64: 4.1e9 bytes), sides of 2D domains at most 2560.
 constexpr int kMidLong = 896;
 template <int N>
 using MidOff = std::conditional_t<(N >= kMidLong), unsigned long, unsigned>;
@@ -301,7 +301,9 @@ hipError_t launch_mid_set(const MidArgs<T>& a0, int n, hipStream_t s) {
         constexpr int NN = decltype(NC)::value;
         if (a.op >= kMidScale) {
             if (single) return launch_k(k_mid<T, NN, 1, true, true>, grid, dim3(thr), smem, s, a);
-            return launch_k(k_mid<T, NN, 1, false, true>, grid, dim3(thr), smem, s, a);
+            // the residual is ImplicitEuler's, which runs in FP64
+            if constexpr (sizeof(T) == 8) return launch_k(k_mid<T, NN, 1, false, true>, grid, dim3(thr), smem, s, a);
+            else return hipErrorInvalidValue;
         }
         if (single) return launch_k(k_mid<T, NN, 1, true, false>, grid, dim3(thr), smem, s, a);
         return launch_k(k_mid<T, NN, 1, false, false>, grid, dim3(thr), smem, s, a);

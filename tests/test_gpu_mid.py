@@ -1,6 +1,7 @@
 """The general path's middle pass (forward, stage, inverse along the last axis in one launch)
 against the oracle: lengths with and without a compiled schedule, one line term and several, terms
-with a LAP power, a constant term, a field's own and another field's spectrum as a term, filter.
+with a LAP power, a constant term, a field's own and another field's spectrum as a term, filter
+(a volume constraint's multiplier: test_gpu_terms.py).
 FP64 to the path's parity bound (1e-10 max relative), FP32 to 1e-5 relative L2.
 """
 import numpy as np
@@ -25,6 +26,9 @@ MODELS = {
     "cross": (["aaa", "bbb"], {"kap": 0.2, "cpl": 0.3}, ["daaa/dt = cpl*bbb + PAA + kap*LAP aaa",
                                                          "dbbb/dt = cpl*aaa - PBB + kap*LAP bbb"],
               {"PAA": [(0.1, {"aaa": 2, "bbb": 0})], "PBB": [(0.2, {"aaa": 0, "bbb": 3})]}),
+    # a bare scalar: the same value at every k, without a brick
+    "constant": (["aaa", "bbb"], {"kap": 0.2, "src": 0.3}, ["daaa/dt = src + PAA + kap*LAP aaa", "dbbb/dt = src - PBB"],
+                 {"PAA": [(0.1, {"aaa": 2, "bbb": 0})], "PBB": [(0.2, {"aaa": 0, "bbb": 3})]}),
 }
 
 
@@ -51,13 +55,11 @@ def pair(name, dims, seed):
     return pm, om, init
 
 
-@pytest.mark.parametrize("filter_order", [0, 4])
+# the filter enters through the factor table only: one model covers it
+@pytest.mark.parametrize("name,filter_order", [(n, 0) for n in sorted(MODELS)] + [("single", 4)])
 @pytest.mark.parametrize("dims", [[9, 15], [2, 16], [40, 24], [100, 12], [12, 400], [11, 11, 11], [24, 24, 24]])
 @pytest.mark.parametrize("stepper", ["euler", "rk4"])
-@pytest.mark.parametrize("name", sorted(MODELS))
-def test_middle_pass_matches_oracle(name, stepper, dims, filter_order):
-    if filter_order and name != "single":
-        pytest.skip("the filter enters through the factor table only: one model covers it")
+def test_middle_pass_matches_oracle(name, filter_order, stepper, dims):
     pm, om, init = pair(name, dims, 5)
     o = E.OracleSolver(om, dims, init, 0.02, stepper, filter_order=filter_order)
     o.solver_propagate(6)
