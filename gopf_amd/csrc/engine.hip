@@ -610,10 +610,12 @@ private:
     // without it).  One wavefront of the next row pass adds up the blocks' partial sums, 64 at a
     // time, and folds the series slot with at least 64 threads: blocks of 256 threads unless they
     // would be fewer than 256 (us a step with blocks of 64 and 128 threads, and of 256: 192^3 FP32
-    // 110.0 and 83.4, FP64 157.0 and 137.8; 256^3 FP64 295 and 273; 128^3 FP32 51.8 and 48.9)
-    int mon_threads(long lines, int per_line) const {
+    // 110.0 and 83.4, FP64 157.0 and 137.8; 256^3 FP64 295 and 273; 128^3 FP32 51.8 and 48.9).
+    // FP64 lines of 28 elements per thread keep 64: their passes spill and take long enough to hide
+    // the sums (224^3 346, with larger blocks 358)
+    int mon_threads(long lines, int per_line, int n) const {
         if (!mon_) return 0;
-        int t = 256;
+        int t = (sizeof(T) == 8 && n / per_line >= 28) ? 64 : 256;
         while (t > 64 && lines * per_line < 256L * t) t /= 2;
         return t;
     }
@@ -1359,7 +1361,7 @@ RowFusedArgs<T> Engine<T>::rows_args(cpx<T>* W, double* mean, int tw, int var) {
     ra.rows = g_.rows;
     ra.nx = g_.nx;
     const long lines = (g_.rows + 1) / 2;
-    ra.TW = tw > 0 ? tw : rows_tw(lines, var, mon_threads(lines, fft_threads_per_line(g_.nx, var)));
+    ra.TW = tw > 0 ? tw : rows_tw(lines, var, mon_threads(lines, fft_threads_per_line(g_.nx, var), g_.nx));
     ra.variant = var;
     ra.c_out = c_out_;
     ra.npoly = (int)fp_.gpoly.size();
@@ -1383,10 +1385,11 @@ PencilUpdateArgs<T> Engine<T>::update_args(cpx<T>* S, cpx<T>* W, double* mean, i
     u.p.seg[1] = (axis == 2) ? seg_z_nyq(g_) : seg_y_nyq(g_);
     u.p.nseg = 2;
     const long lines = pencil_blocks(u.p.seg, u.p.nseg, 1, nullptr);
+    const int mt = mon_threads(lines, fft_threads_per_line(nu, 1), nu);
     u.p.TW = tw > 0 ? tw
                     : fit_tw(nu, sizeof(cpx<T>), 1, true, lines,
                              [&](int t) { return pencil_blocks(u.p.seg, u.p.nseg, t, nullptr); },
-                             mon_threads(lines, fft_threads_per_line(nu, 1)));
+                             mt > 64 ? mt : 0);
     u.g = g_.kg;
     u.dt = dt_;
     u.scale = 1.0 / (double)g_.n;
