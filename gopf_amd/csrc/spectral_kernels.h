@@ -556,13 +556,14 @@ __device__ __forceinline__ void pencil_update_body(UA u, int blk, int nblk, unsi
         }
     } else {
         if constexpr (!EARLY) load_line<T, E>(c, sarr, base, ti.es, lm.t, TT, valid);
-        if constexpr (kApart || !EARLY) {
+        if constexpr (kApart || !EARLY || (MON && sizeof(T) == 4)) {
 #pragma unroll
             for (int e = 0; e < E; ++e) update(e, c[e], s1a[e], gs[e]);
         } else {
             // the same written out: with the call the persistent step's kernel is compiled to other
             // instructions (1000 steps of FP64 128^2 with the energy series, fresh processes in turn:
-            // 13.02 against 12.83 ms; on another card 13.28 against 12.94)
+            // 13.02 against 12.83 ms; on another card 13.28 against 12.94; FP32 the other way with
+            // the series, 13.80 against 14.36, and 10.06 against 9.70 without it)
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 const cpx<T> cv = c[e];
